@@ -240,11 +240,9 @@ struct hh_solver {
   // hierarchy
   bool built = false;
   std::vector<Level> lv;
-  cx<double>* coarse_aug = nullptr;  // n x 2n augmented; right half = inverse
+  cx<double>* coarse_aug = nullptr;  // n x 2n: row-major inverse, then the elimination's workspace
   cx<double>* coarse_d = nullptr;    // coarsest diagonal in complex128
-  int64_t* piv = nullptr;
-  cx<double>* fac = nullptr;
-  cx<double>* pinv = nullptr;
+  char* gj_work = nullptr;           // pivots and row order of the elimination
   float* coarse_pack = nullptr;      // fp32 real-ified inverse for the MFMA apply (complex64 mode)
   int cap = 0;  // RHS capacity of the work buffers
   // Krylov storage
@@ -353,8 +351,8 @@ struct hh_solver {
     free_work();
     for (auto& L : lv) { dfree(L.m); dfree(L.gam); dfree(L.d); dfree(L.f); }
     lv.clear();
-    dfree(coarse_aug); dfree(coarse_d); dfree(piv); dfree(fac); dfree(pinv); dfree(coarse_pack);
-    coarse_aug = nullptr; coarse_d = nullptr; piv = nullptr; fac = nullptr; pinv = nullptr; coarse_pack = nullptr;
+    dfree(coarse_aug); dfree(coarse_d); dfree(gj_work); dfree(coarse_pack);
+    coarse_aug = nullptr; coarse_d = nullptr; gj_work = nullptr; coarse_pack = nullptr;
     built = false;
     learn_verdict = -1;
   }
@@ -447,10 +445,8 @@ void build_hierarchy(hh_solver* S) {
   S->coarse_d = dalloc<cx<double>>(n);
   launch_diag<double>(c.g, c.m, c.gam, op->wre, op->wim, op->neumann_top, op->sommerfeld, c.h, S->coarse_d, st);
   S->coarse_aug = dalloc<cx<double>>((size_t)n * 2 * n);
-  S->piv = dalloc<int64_t>(1);
-  S->fac = dalloc<cx<double>>(n);
-  S->pinv = dalloc<cx<double>>(1);
-  launch_dense_inverse(c.g, S->coarse_d, S->coarse_aug, S->piv, S->fac, S->pinv, st);
+  S->gj_work = dalloc<char>(dense_inverse_work_bytes(n));
+  launch_dense_inverse(c.g, S->coarse_d, S->coarse_aug, S->gj_work, st);
   if (S->p.prec == HH_C64) {
     // complex64 preconditioner: the coarsest apply runs on MFMA from an fp32 copy
     S->coarse_pack = dalloc<float>((size_t)pack_inv_mfma_size(c.g.N));

@@ -36,9 +36,9 @@ template <typename T>
 void launch_jacobi_factor(const Grid& g, const double* m, const double* gam, double wre, double wim, int neumann_top,
                           int sommerfeld, const double h[3], double relax, cx<T>* f, hipStream_t s);
 void launch_add_const(double* a, double c, int64_t n, hipStream_t s);
-// leaves A^-1 row-major in M[0, n*n) (and column-major in M[n*n, 2*n*n))
-void launch_dense_inverse(const Grid& g, const cx<double>* d, cx<double>* M, int64_t* piv, cx<double>* fac,
-                          cx<double>* pinv, hipStream_t s);
+// leaves A^-1 row-major in M[0, n*n); M[n*n, 2*n*n) and work (dense_inverse_work_bytes(n) bytes) are its workspace
+size_t dense_inverse_work_bytes(int64_t n);
+void launch_dense_inverse(const Grid& g, const cx<double>* d, cx<double>* M, void* work, hipStream_t s);
 template <typename T>
 void launch_dense_apply(const cx<double>* Ainv, int64_t n, int nrhs, const cx<T>* r, cx<T>* x, const int* skip,
                         hipStream_t s);

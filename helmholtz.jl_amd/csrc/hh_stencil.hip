@@ -434,116 +434,7 @@ __global__ __launch_bounds__(256) void k_add_const(double* __restrict__ a, doubl
   if (p < n) a[p] += c;
 }
 
-// ---- coarsest level: dense operator, Gauss-Jordan inverse, dense apply ----
-// Column-major n x 2n augmented matrix [A | I]; after elimination the right
-// half holds A^-1.
-__global__ __launch_bounds__(256) void k_dense_assemble(Grid g, const cx<double>* __restrict__ d,
-                                                        cx<double>* __restrict__ M) {
-  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t n = g.N;
-  if (p >= n) return;
-  const int i = (int)(p % g.n1);
-  const int64_t q = p / g.n1;
-  const int j = (int)(q % g.n2);
-  const int k = (int)(q / g.n2);
-  const int64_t P1 = g.n1, P2 = (int64_t)g.n1 * g.n2;
-  // row p of A: sum_d ih_d (2 x_p - x_lo - x_hi) + d_p x_p
-  double diag = 2.0 * (g.ih1 + g.ih2 + (g.dim == 3 ? g.ih3 : 0.0));
-  M[p + p * n] = mk<double>(diag + d[p].re, d[p].im);
-  int64_t nb[6];
-  double cf[6];
-  int cnt = 0;
-  nb[cnt] = (int64_t)k * P2 + j * P1 + lo_nb(i, g.bc); cf[cnt++] = g.ih1;
-  nb[cnt] = (int64_t)k * P2 + j * P1 + hi_nb(i, g.n1, g.bc); cf[cnt++] = g.ih1;
-  nb[cnt] = (int64_t)k * P2 + lo_nb(j, g.bc) * P1 + i; cf[cnt++] = g.ih2;
-  nb[cnt] = (int64_t)k * P2 + hi_nb(j, g.n2, g.bc) * P1 + i; cf[cnt++] = g.ih2;
-  if (g.dim == 3) {
-    nb[cnt] = (int64_t)lo_nb(k, g.bc) * P2 + j * P1 + i; cf[cnt++] = g.ih3;
-    nb[cnt] = (int64_t)hi_nb(k, g.n3, g.bc) * P2 + j * P1 + i; cf[cnt++] = g.ih3;
-  }
-  for (int c = 0; c < cnt; ++c) {
-    cx<double>& e = M[p + nb[c] * n];
-    e.re -= cf[c];
-  }
-  M[p + (n + p) * n] = mk<double>(1.0, 0.0);
-}
-
-// pivot search in column k (rows k..n-1): one block of 256 threads; stores
-// the pivot row and the reciprocal of the pivot value.
-__global__ __launch_bounds__(256) void k_gj_pivot(const cx<double>* __restrict__ M, int64_t n, int64_t k,
-                                                  int64_t* __restrict__ piv, cx<double>* __restrict__ pinv) {
-  __shared__ double sv[256];
-  __shared__ int64_t si[256];
-  double best = -1.0;
-  int64_t bi = k;
-  for (int64_t r = k + threadIdx.x; r < n; r += 256) {
-    double v = cabs2(M[r + k * n]);
-    if (v > best) { best = v; bi = r; }
-  }
-  sv[threadIdx.x] = best;
-  si[threadIdx.x] = bi;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) {
-      double o = sv[threadIdx.x + s];
-      int64_t oi = si[threadIdx.x + s];
-      if (o > sv[threadIdx.x] || (o == sv[threadIdx.x] && oi < si[threadIdx.x])) {
-        sv[threadIdx.x] = o;
-        si[threadIdx.x] = oi;
-      }
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    piv[0] = si[0];
-    pinv[0] = cinv(M[si[0] + k * n]);
-  }
-}
-
-// elimination factors of column k as they stand after the row swap k <-> piv
-__global__ __launch_bounds__(256) void k_gj_fac(const cx<double>* __restrict__ M, int64_t n, int64_t k,
-                                                const int64_t* __restrict__ piv, cx<double>* __restrict__ fac) {
-  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (r >= n) return;
-  const int64_t pr = piv[0];
-  cx<double> f = (r == pr) ? M[k + k * n] : M[r + k * n];
-  if (r == k) f = mk<double>(0.0, 0.0);
-  fac[r] = f;
-}
-
-// swap rows k and piv and scale the new row k; one thread per column
-__global__ __launch_bounds__(256) void k_gj_swap_scale(cx<double>* __restrict__ M, int64_t n, int64_t k,
-                                                       const int64_t* __restrict__ piv,
-                                                       const cx<double>* __restrict__ pinv) {
-  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (c >= 2 * n) return;
-  const int64_t pr = piv[0];
-  const cx<double> a = M[k + c * n];
-  const cx<double> b = M[pr + c * n];
-  if (pr != k) M[pr + c * n] = a;
-  M[k + c * n] = b * pinv[0];
-}
-
-__global__ __launch_bounds__(256) void k_gj_elim(cx<double>* __restrict__ M, int64_t n, int64_t k,
-                                                 const cx<double>* __restrict__ fac) {
-  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t c = (int64_t)blockIdx.y + k;  // columns k..2n-1
-  if (r >= n || c >= 2 * n || r == k) return;
-  cx<double> f = fac[r];
-  if (f.re == 0.0 && f.im == 0.0) return;
-  M[r + c * n] = M[r + c * n] - f * M[k + c * n];
-}
-
-// After elimination the left half of [A | I] is the identity and the right
-// half is A^-1 (column-major); copy A^-1 row-major into the left half so a
-// row is contiguous for the apply below.
-__global__ __launch_bounds__(256) void k_inv_rows(cx<double>* __restrict__ M, int64_t n) {
-  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (k >= n * n) return;
-  const int64_t i = k / n, j = k - i * n;
-  M[k] = M[n * n + j * n + i];
-}
-
+// ---- coarsest level: apply of the dense inverse (hh_dense.hip) ----
 // x_b = Ainv r_b in complex128 for every right-hand side.  One wavefront per
 // RT rows and DR right-hand sides: lanes stride the columns of the row-major
 // inverse (coalesced), each lane keeps RT x DR partial sums, wave shuffles
@@ -846,22 +737,6 @@ template void launch_jacobi_factor<float>(const Grid&, const double*, const doub
 
 void launch_add_const(double* a, double c, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_add_const, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, c, n);
-}
-
-void launch_dense_inverse(const Grid& g, const cx<double>* d, cx<double>* M, int64_t* piv, cx<double>* fac,
-                          cx<double>* pinv, hipStream_t s) {
-  const int64_t n = g.N;
-  hipMemsetAsync(M, 0, sizeof(cx<double>) * n * 2 * n, s);
-  hipLaunchKernelGGL(k_dense_assemble, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g, d, M);
-  for (int64_t k = 0; k < n; ++k) {
-    hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(256), 0, s, M, n, k, piv, pinv);
-    hipLaunchKernelGGL(k_gj_fac, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, M, n, k, piv, fac);
-    hipLaunchKernelGGL(k_gj_swap_scale, dim3((unsigned)((2 * n + 255) / 256)), dim3(256), 0, s, M, n, k, piv,
-                       pinv);
-    hipLaunchKernelGGL(k_gj_elim, dim3((unsigned)((n + 255) / 256), (unsigned)(2 * n - k)), dim3(256), 0, s, M, n,
-                       k, fac);
-  }
-  hipLaunchKernelGGL(k_inv_rows, dim3((unsigned)((n * n + 255) / 256)), dim3(256), 0, s, M, n);
 }
 
 template <typename T>
