@@ -14,11 +14,13 @@
 //                exchanges to them and adds panel * M_KJ.
 // Panels of NBI columns are grouped NB = 32 to a block: inside a block only
 // the block's own columns are updated (rank NBI), the rest of the matrix once
-// per block (rank 32).  The rank-1 form it replaces (four launches and one pass
-// over n x 1.5 n values per column) was bound by launches for n ~ 500 and by
-// those passes for n ~ 2000.  Whole set-up of a solver on MI355X before / after
-// (hierarchy included): 561 nodes 11.7 / @561@ ms, 1183 nodes 30.6 / @1183@ ms,
-// 2145 nodes 72.7 / @2145@ ms, 8385 nodes 2950 / @8385@ ms.
+// once per block (rank 32).  The rank-1 form it replaces (four launches and one
+// pass over n x 1.5 n values per column) was bound by launches for n ~ 500 and
+// by those passes for n ~ 2000; this one is bound by the panels' serial chain
+// (15-16 us per panel of 8, 6 or 4 columns) and, for n > 2000, by the rank-32
+// updates as well.  Set-up time of a solver on MI355X (hierarchy included),
+// rank-1 form / this one: 561 nodes 7.0 / 2.0 ms, 1183 nodes 23.5 / 7.0 ms,
+// 2145 nodes 62 / 17 ms, 8385 nodes 2943 / 371 ms.
 #include <algorithm>
 
 #include "hh_kernels.h"
@@ -111,8 +113,8 @@ __device__ __forceinline__ unsigned long long wave_max(unsigned long long v) {
 // pout (with the block's last panel, else null): the whole block's exchange.
 // A pivot is found as the maximum of one 64-bit key per row, |a|^2 with its 14
 // lowest bits (6e-13 of it, n < 2^14) replaced by the reversed row number: one
-// DPP reduction and one LDS atomic per wavefront.  One column takes about 1.3 us
-// of the panel's time (5 us with value and row reduced by shuffles).
+// DPP reduction and one LDS atomic per wavefront (a 4-column panel of 2145 rows:
+// 20 us with value and row reduced by shuffles, 15 us so).
 template <int W, int R>
 __global__ __launch_bounds__(1024) void k_gj_panel(cx<double>* __restrict__ M, int n, int k0, int w, int kb,
                                                    int* __restrict__ piv, GjPerm* __restrict__ pin,
