@@ -14,7 +14,7 @@
 //                exchanges to them and adds panel * M_KJ.
 // Panels of NBI columns are grouped NB = 32 to a block: inside a block only
 // the block's own columns are updated (rank NBI), the rest of the matrix once
-// once per block (rank 32).  The rank-1 form it replaces (four launches and one
+// per block (rank 32).  The rank-1 form it replaces (four launches and one
 // pass over n x 1.5 n values per column) was bound by launches for n ~ 500 and
 // by those passes for n ~ 2000; this one is bound by the panels' serial chain
 // (15-16 us per panel of 8, 6 or 4 columns) and, for n > 2000, by the rank-32

@@ -438,34 +438,57 @@ __global__ __launch_bounds__(256) void k_add_const(double* __restrict__ a, doubl
 // x_b = Ainv r_b in complex128 for every right-hand side.  One wavefront per
 // RT rows and DR right-hand sides: lanes stride the columns of the row-major
 // inverse (coalesced), each lane keeps RT x DR partial sums, wave shuffles
-// combine them.  The inverse is re-read nrhs/DR times and r n/RT times.
-constexpr int DR = 4, RT = 4;
-template <typename T>
-__global__ __launch_bounds__(256) void k_dense_apply(const cx<double>* __restrict__ Arow, int64_t n, int nrhs,
+// combine them (the same order of additions for every RT and DR).  The inverse
+// is re-read nrhs/DR times and r n/RT times.  UN column steps are loaded before
+// the first is used: with few right-hand sides a wavefront reads one or two rows
+// and nothing else hides the loads' latency.
+template <typename T, int RT, int DR, int UN>
+__global__ __launch_bounds__(256) void k_dense_apply(const cx<double>* __restrict__ Arow, int n, int nrhs,
                                                      const cx<T>* __restrict__ r, cx<T>* __restrict__ x,
                                                      const int* __restrict__ skip) {
   const int lane = threadIdx.x & 63;
-  const int64_t i0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RT;
+  const int i0 = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * RT;
   const int rhs0 = blockIdx.y * DR;
   if (i0 >= n) return;  // uniform per wavefront
   const int nr = min(DR, nrhs - rhs0);
-  const int ni = (int)min((int64_t)RT, n - i0);
+  const int ni = min(RT, n - i0);
+  bool live = !skip;
+  for (int k = 0; k < nr && !live; ++k) live = !skip[rhs0 + k];
+  if (!live) return;
+  const cx<double>* row[RT];
+#pragma unroll
+  for (int a = 0; a < RT; ++a) row[a] = Arow + (int64_t)min(i0 + a, n - 1) * n;
+  const cx<T>* rc[DR];
+#pragma unroll
+  for (int k = 0; k < DR; ++k) rc[k] = r + (int64_t)(rhs0 + min(k, nr - 1)) * n;
   cx<double> acc[RT][DR];
 #pragma unroll
   for (int a = 0; a < RT; ++a)
 #pragma unroll
     for (int k = 0; k < DR; ++k) acc[a][k] = mk<double>(0.0, 0.0);
-  for (int64_t j = lane; j < n; j += 64) {
-    cx<double> rv[DR];
+  int j = lane;
+  for (; j + 64 * (UN - 1) < n; j += 64 * UN) {
+    cx<double> av[UN][RT], rv[UN][DR];
 #pragma unroll
-    for (int k = 0; k < DR; ++k)
-      rv[k] = k < nr ? cvt<T, double>(r[(int64_t)(rhs0 + k) * n + j]) : mk<double>(0.0, 0.0);
+    for (int u = 0; u < UN; ++u) {
+#pragma unroll
+      for (int a = 0; a < RT; ++a) av[u][a] = row[a][j + 64 * u];
+#pragma unroll
+      for (int k = 0; k < DR; ++k) rv[u][k] = cvt<T, double>(rc[k][j + 64 * u]);
+    }
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+#pragma unroll
+      for (int a = 0; a < RT; ++a)
+#pragma unroll
+        for (int k = 0; k < DR; ++k) acc[a][k] = acc[a][k] + av[u][a] * rv[u][k];
+  }
+  for (; j < n; j += 64) {
 #pragma unroll
     for (int a = 0; a < RT; ++a) {
-      if (a >= ni) break;
-      const cx<double> av = Arow[(i0 + a) * n + j];
+      const cx<double> av = row[a][j];
 #pragma unroll
-      for (int k = 0; k < DR; ++k) acc[a][k] = acc[a][k] + av * rv[k];
+      for (int k = 0; k < DR; ++k) acc[a][k] = acc[a][k] + av * cvt<T, double>(rc[k][j]);
     }
   }
 #pragma unroll
@@ -739,11 +762,33 @@ void launch_add_const(double* a, double c, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_add_const, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, c, n);
 }
 
+template <typename T, int RT, int DR, int UN>
+static void dense_apply_go(const cx<double>* Ainv, int n, int nrhs, const cx<T>* r, cx<T>* x, const int* skip,
+                           hipStream_t s) {
+  dim3 grid((unsigned)((n + 4 * RT - 1) / (4 * RT)), (unsigned)((nrhs + DR - 1) / DR));
+  hipLaunchKernelGGL((k_dense_apply<T, RT, DR, UN>), grid, dim3(256), 0, s, Ainv, n, nrhs, r, x, skip);
+}
+
+// 4 rows x 4 RHS per wavefront read the inverse and r least often, but leave
+// 561 rows x 1 RHS with 36 blocks, three of whose four sums are padding: below
+// 1200 such wavefronts a wavefront takes one row and up to four RHS, and a single
+// RHS always has the one-row form.  Measured on MI355X, 4 x 4 form / this one,
+// with 14 us of copies and call around each: 561 nodes 1 RHS 26 / 18 us, 4 RHS
+// 28 / 20; 1183 nodes 8 RHS 36 / 28; 2145 nodes 1 RHS 44 / 29, 4 RHS 47 / 36,
+// 8 RHS 51 / 50; beyond the line 2145 nodes 12 RHS 56 / 62, 6305 nodes 2 RHS
+// 138 / 166.  6305 nodes 1 RHS: 134 / 134, the inverse at 5.3 TB/s.
 template <typename T>
 void launch_dense_apply(const cx<double>* Ainv, int64_t n, int nrhs, const cx<T>* r, cx<T>* x, const int* skip,
                         hipStream_t s) {
-  dim3 grid((unsigned)((n + 4 * RT - 1) / (4 * RT)), (unsigned)((nrhs + DR - 1) / DR));
-  hipLaunchKernelGGL((k_dense_apply<T>), grid, dim3(256), 0, s, Ainv, n, nrhs, r, x, skip);
+  const int64_t waves = ((n + 3) / 4) * ((nrhs + 3) / 4);
+  if (nrhs == 1)
+    dense_apply_go<T, 1, 1, 8>(Ainv, (int)n, nrhs, r, x, skip, s);
+  else if (waves >= 1200)
+    dense_apply_go<T, 4, 4, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
+  else if (nrhs == 2)
+    dense_apply_go<T, 1, 2, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
+  else
+    dense_apply_go<T, 1, 4, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
 }
 template void launch_dense_apply<double>(const cx<double>*, int64_t, int, const cx<double>*, cx<double>*,
                                          const int*, hipStream_t);

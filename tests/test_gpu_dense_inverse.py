@@ -46,3 +46,27 @@ def test_inverse_needs_pivoting(nodes, omega):
     A = hr.operator_from_param(hr.HelmholtzParam(M, g, m, w, True, True), 2).toarray()
     Z = ha.precondition(s, np.eye(N, dtype=complex))
     assert np.linalg.norm(Z - np.linalg.inv(A)) <= 64 * N * EPS * np.linalg.cond(A) * np.linalg.norm(np.linalg.inv(A))
+
+
+# one row per wavefront with 1, 2 and 4 right-hand sides (remainders of 4, of 64
+# and of the 256 / 512 columns loaded at a time), and the 4 x 4 tiles
+@pytest.mark.parametrize("nodes,nrhs", [((3, 3), 1), ((8, 8), 1), ((21, 25), 1), ((33, 17), 1), ((33, 17), 2), ((33, 17), 3),
+                                        ((33, 17), 4), ((33, 17), 9), ((23, 23), 7), ((33, 17), 35), ((65, 33), 8),
+                                        ((65, 33), 9)])
+def test_apply_tiles(nodes, nrhs):
+    """Column c of a block does not depend on the tile it falls into: the sums run
+    in one order for every tile, so each column equals the same column alone."""
+    import helmholtz_amd as ha
+    from problems import small_case
+    M, m, g, w = small_case(nodes, seed=3)
+    hp = ha.HelmholtzParam(ha.getRegularMesh(M.domain, M.n), g, m, w, True, True)
+    mg = ha.getMGparam(complex, int, 1, 1, 1, 1e-6, "Jac", 0.8, 2, 2, "V", "NoMUMPS", 0.5, 0.0)
+    s = ha.getShiftedLaplacianMultigridSolver(hp, mg, 0.5, "GMRES", 2)
+    N = int(np.prod(nodes))
+    rng = np.random.default_rng(4)
+    V = rng.standard_normal((N, nrhs)) + 1j * rng.standard_normal((N, nrhs))
+    Z = ha.precondition(s, V)
+    inv = ha.precondition(s, np.eye(N, dtype=complex))
+    assert np.linalg.norm(Z - inv @ V) <= 8 * N * EPS * np.linalg.norm(inv) * np.linalg.norm(V)
+    for c in {0, nrhs // 2, nrhs - 1}:
+        assert np.array_equal(ha.precondition(s, V[:, [c]])[:, 0], Z[:, c])
