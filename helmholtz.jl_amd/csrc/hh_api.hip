@@ -547,10 +547,19 @@ void ensure_work(hh_solver* S, int nrhs) {
   w.nrhs = nrhs;
   w.N = N;
   w.kmax = K;
-  // node chunks per RHS for the Arnoldi/BiCGSTAB reductions: about 16K
-  // blocks in all (64 per CU, so the last wave of blocks is a small tail),
-  // chunks of at least 4096 nodes
-  int nchunk = (int)std::max<int64_t>(1, std::min<int64_t>((16384 + nrhs - 1) / nrhs, (N + 4095) / 4096));
+  // Node chunks per RHS for the Arnoldi/BiCGSTAB reductions: about 16K blocks
+  // in all (64 per CU, so the last wave of blocks is a small tail), chunks of at
+  // least `least` nodes.  That is 1/1024 of the grid between 256 nodes (one per
+  // thread) and 4096, so one RHS alone still spreads over the chip: with chunks
+  // of 4096 nodes the passes of a 129 x 129 grid ran on 5 blocks (pass 1 at 10
+  // vectors 35 us, pass 2 29 us, against 5.7 and 6.1) and those of 1025 x 513 on
+  // 129 (55 and 58 us against 17 and 20).  It depends on the grid only, not
+  // on the number of RHS, so a small block gives the bits of single solves.  Where
+  // the passes carry a window of 2 n1 extra values of z (complex64 cycle) a chunk
+  // is at least twice that.
+  int64_t least = std::min<int64_t>(4096, std::max<int64_t>(256, ((N + 1023) / 1024 + 255) / 256 * 256));
+  if (pr == HH_C64) least = std::min<int64_t>(4096, std::max<int64_t>(least, 4 * (int64_t)S->lv[0].g.n1));
+  int nchunk = (int)std::max<int64_t>(1, std::min<int64_t>((16384 + nrhs - 1) / nrhs, (N + least - 1) / least));
   // 3-D: chunk c is in-plane segment c mod nseg3 over run c / nseg3 of the
   // planes (runs of at least 8 planes) for the H z passes' z march
   w.nseg3 = 0;

@@ -45,6 +45,37 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
   return r;
 }
 
+// Sums of M values over a wavefront, the values shared out among the lanes as
+// the reduction narrows: at each step a lane keeps one half of its values and
+// hands the other half to its partner, so M = 21 takes 23 exchanges where M
+// separate reductions take 126 (the same tree of additions, the same bits).
+// On return v[0 .. K) holds the sums of values base .. base + valid - 1.
+template <int M, int O>
+struct WaveSums {
+  static constexpr int Hf = (M + 1) / 2;
+  template <typename F>
+  static __device__ __forceinline__ void run(const double (&v)[M], int lane, int base, int valid, F&& put) {
+    double h[Hf];
+    const bool hi = (lane & O) != 0;
+#pragma unroll
+    for (int k = 0; k < Hf; ++k) {
+      const double up = k + Hf < M ? v[k + Hf < M ? k + Hf : 0] : 0.0;
+      const double send = M > 1 && hi ? v[k] : up, keep = M > 1 && hi ? up : v[k];
+      h[k] = keep + __shfl_xor(M > 1 ? send : v[k], O, 64);
+    }
+    if (M > 1) {
+      base = hi ? base + Hf : base;
+      valid = hi ? valid - Hf : min(valid, Hf);
+    }
+    if constexpr (O > 1)
+      WaveSums<Hf, O / 2>::run(h, lane, base, valid, put);
+    else
+#pragma unroll
+      for (int k = 0; k < Hf; ++k)
+        if (k < valid) put(base + k, h[k]);
+  }
+};
+
 static __device__ __forceinline__ void chunk_range(int64_t N, int nchunk, int c, int64_t* a, int64_t* b) {
   const int64_t L = (N + nchunk - 1) / nchunk;
   *a = (int64_t)c * L;
@@ -66,6 +97,33 @@ __device__ __forceinline__ cx<double> csub_mul(cx<double> w, cx<double> h, cx<do
 // nn + |w|^2
 __device__ __forceinline__ double nrm_acc(double nn, cx<double> w) { return fma(w.im, w.im, fma(w.re, w.re, nn)); }
 
+// Block sums (256 threads) of acc[0..j] (times the basis scale in lazy mode) into
+// part[c][i][b] and, with NORM, of nn into partn[c][b].
+template <int NV, bool NORM>
+__device__ __forceinline__ void store_sums(const KrylovWork& kw, int c, int b, int j, const cx<double> (&acc)[NV],
+                                           double nn) {
+  constexpr int M = 2 * NV + (NORM ? 1 : 0);
+  __shared__ double sums[4][M];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  double v[M];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const double si = kw.lazy && i <= j ? kw.vscale[i * kw.nrhs + b] : 1.0;
+    v[2 * i] = si * acc[i].re;
+    v[2 * i + 1] = si * acc[i].im;
+  }
+  if (NORM) v[M - 1] = nn;
+  WaveSums<M, 32>::run(v, lane, 0, M, [&](int q, double s) { sums[wid][q] = s; });
+  __syncthreads();
+  const int q = threadIdx.x;
+  if (q >= M) return;
+  const double s = ((sums[0][q] + sums[1][q]) + sums[2][q]) + sums[3][q];
+  if (NORM && q == M - 1)
+    kw.partn[(int64_t)c * kw.nrhs + b] = s;
+  else if (q < 2 * (j + 1))
+    ((double*)kw.part)[2 * (((int64_t)c * (kw.kmax + 1) + (q >> 1)) * kw.nrhs + b) + (q & 1)] = s;
+}
+
 // pass 1: part[c][i][b] = sum_{p in chunk c} conj(V_i[p,b]) w[p,b], i <= j
 // NORM: also partn[c][b] = sum ||w||^2 over the chunk.  only (may be null):
 // skip RHS with only[b] == 0.
@@ -75,7 +133,6 @@ __global__ __launch_bounds__(256) void k_dots(KrylovWork kw, const cx<TV>* __res
                                               const int* __restrict__ only) {
   const int c = blockIdx.x, b = blockIdx.y;
   if (kw.done[b] || (only && !only[b])) return;
-  __shared__ double sh[4];
   int64_t p0, p1;
   chunk_range(kw.N, kw.nchunk, c, &p0, &p1);
   const int64_t stride = kw.N * kw.nrhs;
@@ -86,24 +143,39 @@ __global__ __launch_bounds__(256) void k_dots(KrylovWork kw, const cx<TV>* __res
   double nn = 0.0;
   for (int64_t p = p0 + threadIdx.x; p < p1; p += 256) {
     const cx<double> wv = cvt<TV, double>(w[base + p]);
-    if (NORM) nn = nrm_acc(nn, wv);
+    if constexpr (NV <= 10) {
+      // every load before the first use; basis vector j stands in for those past it
+      cx<TV> vv[NV];
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
-      if (i <= j) acc[i] = cmac_conj(acc[i], cvt<TV, double>(V[i * stride + base + p]), wv);
-  }
+      for (int i = 0; i < NV; ++i) vv[i] = V[min(i, j) * stride + base + p];
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    if (i <= j) {  // (no early exit: keeps acc[] in registers)
-      const double si = kw.lazy ? kw.vscale[i * kw.nrhs + b] : 1.0;
-      const double re = block_sum(si * acc[i].re, sh);
-      const double im = block_sum(si * acc[i].im, sh);
-      if (threadIdx.x == 0) kw.part[((int64_t)c * (kw.kmax + 1) + i) * kw.nrhs + b] = mk<double>(re, im);
+      for (int i = 0; i < NV; ++i) acc[i] = cmac_conj(acc[i], cvt<TV, double>(vv[i]), wv);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        if (i <= j) acc[i] = cmac_conj(acc[i], cvt<TV, double>(V[i * stride + base + p]), wv);
     }
+    if (NORM) nn = nrm_acc(nn, wv);
   }
-  if (NORM) {
-    const double t = block_sum(nn, sh);
-    if (threadIdx.x == 0) kw.partn[(int64_t)c * kw.nrhs + b] = t;
+  store_sums<NV, NORM>(kw, c, b, j, acc, nn);
+}
+
+// a lane's share of the partial sums of (i, b): chunks lane, lane + 64, ... in
+// order, eight of them loaded before the first is added
+__device__ __forceinline__ void chunk_sum(const KrylovWork& kw, int i, int b, int lane, double* re, double* im) {
+  const int64_t step = (int64_t)64 * (kw.kmax + 1) * kw.nrhs;
+  const cx<double>* q = kw.part + ((int64_t)lane * (kw.kmax + 1) + i) * kw.nrhs + b;
+  double r = 0.0, m = 0.0;
+  for (int c = lane; c < kw.nchunk; c += 512) {
+    cx<double> v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = c + 64 * u < kw.nchunk ? q[u * step] : mk<double>(0.0, 0.0);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) r += v[u].re, m += v[u].im;
+    q += 8 * step;
   }
+  *re = r;
+  *im = m;
 }
 
 // reduce part over chunks into h[i][b] (one wavefront per (i, b)); block
@@ -118,12 +190,8 @@ __global__ __launch_bounds__(64) void k_reduce_dots(KrylovWork kw, cx<double>* _
     if (threadIdx.x == 0) kw.wn2[b] = nn;
     return;
   }
-  double re = 0.0, im = 0.0;
-  for (int c = threadIdx.x; c < kw.nchunk; c += 64) {
-    const cx<double> v = kw.part[((int64_t)c * (kw.kmax + 1) + i) * kw.nrhs + b];
-    re += v.re;
-    im += v.im;
-  }
+  double re, im;
+  chunk_sum(kw, i, b, threadIdx.x, &re, &im);
   re = wave_sum(re);
   im = wave_sum(im);
   if (threadIdx.x == 0) {
@@ -142,7 +210,6 @@ __global__ __launch_bounds__(256) void k_update_dots(KrylovWork kw, const cx<dou
                                                      const cx<double>* w, cx<double>* wout, int j) {
   const int c = blockIdx.x, b = blockIdx.y;
   if (kw.done[b]) return;
-  __shared__ double sh[4];
   int64_t p0, p1;
   chunk_range(kw.N, kw.nchunk, c, &p0, &p1);
   const int64_t stride = kw.N * kw.nrhs;
@@ -156,28 +223,18 @@ __global__ __launch_bounds__(256) void k_update_dots(KrylovWork kw, const cx<dou
   for (int64_t p = p0 + threadIdx.x; p < p1; p += 256) {
     cx<double> vv[NV];
     cx<double> wv = w[base + p];
+    // every load before the first use; basis vector j stands in for those past it
+#pragma unroll
+    for (int i = 0; i < NV; ++i) vv[i] = V[min(i, j) * stride + base + p];
 #pragma unroll
     for (int i = 0; i < NV; ++i)
-      if (i <= j) {
-        vv[i] = V[i * stride + base + p];
-        wv = wv - hc[i * hstride] * vv[i];
-      }
+      if (i <= j) wv = wv - hc[i * hstride] * vv[i];
     wout[base + p] = wv;
     nn += cabs2(wv);
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
-      if (i <= j) acc[i] = acc[i] + cmulc(vv[i], wv);
+    for (int i = 0; i < NV; ++i) acc[i] = acc[i] + cmulc(vv[i], wv);
   }
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    if (i <= j) {
-      const double re = block_sum(acc[i].re, sh);
-      const double im = block_sum(acc[i].im, sh);
-      if (threadIdx.x == 0) kw.part[((int64_t)c * (kw.kmax + 1) + i) * kw.nrhs + b] = mk<double>(re, im);
-    }
-  }
-  const double t = block_sum(nn, sh);
-  if (threadIdx.x == 0) kw.partn[(int64_t)c * kw.nrhs + b] = t;
+  store_sums<NV, true>(kw, c, b, j, acc, nn);
 }
 
 // lazy pass 2: w' = w - V h1 (basis vectors carry their scale), partn = ||w'||^2
@@ -346,7 +403,6 @@ __global__ __launch_bounds__(256) void k_dots_hz(KrylovWork kw, Grid g, const cx
   constexpr int S = 256 * U;
   const int b = blockIdx.x, c = blockIdx.y;
   if (kw.done[b]) return;
-  __shared__ double sh[4];
   extern __shared__ cx<float> zr[];
   int64_t p0, p1;
   chunk_range(kw.N, kw.nchunk, c, &p0, &p1);
@@ -422,17 +478,7 @@ __global__ __launch_bounds__(256) void k_dots_hz(KrylovWork kw, Grid g, const cx
       __syncthreads();
     }
   }
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    if (i <= j) {
-      const double si = kw.vscale[i * kw.nrhs + b];
-      const double re = block_sum(si * acc[i].re, sh);
-      const double im = block_sum(si * acc[i].im, sh);
-      if (threadIdx.x == 0) kw.part[((int64_t)c * (kw.kmax + 1) + i) * kw.nrhs + b] = mk<double>(re, im);
-    }
-  }
-  const double t = block_sum(nn, sh);
-  if (threadIdx.x == 0) kw.partn[(int64_t)c * kw.nrhs + b] = t;
+  store_sums<NV, true>(kw, c, b, j, acc, nn);
 }
 
 // pass 2: w' = H z - V h1 (stored in the basis precision), partn = ||w'||^2
@@ -598,7 +644,6 @@ __global__ __launch_bounds__(256) void k_dots_hz3c(KrylovWork kw, Grid g, const 
   constexpr int PT = C3_LQ / 256;  // in-plane nodes per thread (two, taken in turn)
   const int b = blockIdx.x, c = blockIdx.y;
   if (kw.done[b]) return;
-  __shared__ double sh[4];
   extern __shared__ cx<float> zw[];
   const Col3 cb = col3_of(g, c, kw.nseg3);
   const int64_t plane = (int64_t)g.n1 * g.n2;
@@ -664,17 +709,7 @@ __global__ __launch_bounds__(256) void k_dots_hz3c(KrylovWork kw, Grid g, const 
     }
     __syncthreads();
   }
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    if (i <= j) {
-      const double si = kw.vscale[i * kw.nrhs + b];
-      const double re = block_sum(si * acc[i].re, sh);
-      const double im = block_sum(si * acc[i].im, sh);
-      if (threadIdx.x == 0) kw.part[((int64_t)c * (kw.kmax + 1) + i) * kw.nrhs + b] = mk<double>(re, im);
-    }
-  }
-  const double t = block_sum(nn, sh);
-  if (threadIdx.x == 0) kw.partn[(int64_t)c * kw.nrhs + b] = t;
+  store_sums<NV, true>(kw, c, b, j, acc, nn);
 }
 
 // pass 2 (3-D columns): w' = H z - V h1 (stored in the basis precision),
@@ -774,63 +809,79 @@ __global__ __launch_bounds__(64) void k_fix_flags(KrylovWork kw) {
 }
 
 // Reduce pass-2 sums, form column j of H, apply/update Givens rotations and
-// the residual estimate; one wavefront per RHS.
-__global__ __launch_bounds__(64) void k_hess_givens(KrylovWork kw, int j, double tol) {
+// the residual estimate; one block per RHS, its four wavefronts reduce the j + 2
+// sums side by side and the small vectors (the rotations, h1) are read into LDS
+// at the same time.  One wavefront reducing them in turn and walking the
+// rotations through memory took 8.1 us a step at 5 chunks (129 x 129, one RHS);
+// this takes 5.2 us at 65.
+// skip_before[b] = done[b] as it stood before this step.
+__global__ __launch_bounds__(256) void k_hess_givens(KrylovWork kw, int j, double tol,
+                                                     int* __restrict__ skip_before) {
   const int b = blockIdx.x;
-  if (kw.done[b]) return;
-  const int lane = threadIdx.x;
-  __shared__ cx<double> col[72];
-  // h2 and ||w'||^2 (lazy mode: h2 exists only where fix[b] was raised)
-  const bool have_h2 = !kw.lazy || kw.fix[b];
-  double s2 = 0.0;
-  for (int i = 0; i <= j; ++i) {
-    if (!have_h2) {
-      if (lane == 0) col[i] = kw.h1[i * kw.nrhs + b];
-      continue;
-    }
-    double re = 0.0, im = 0.0;
-    for (int c = lane; c < kw.nchunk; c += 64) {
-      const cx<double> v = kw.part[((int64_t)c * (kw.kmax + 1) + i) * kw.nrhs + b];
-      re += v.re;
-      im += v.im;
-    }
-    re = wave_sum(re);
-    im = wave_sum(im);
-    if (lane == 0) {
-      const cx<double> h2 = mk<double>(re, im);
-      kw.h2[i * kw.nrhs + b] = h2;
-      col[i] = kw.h1[i * kw.nrhs + b];
-      s2 += cabs2(h2);
-    }
-  }
-  double nn = 0.0;
-  for (int c = lane; c < kw.nchunk; c += 64) nn += kw.partn[(int64_t)c * kw.nrhs + b];
-  nn = wave_sum(nn);
-  if (lane != 0) return;
-  // the Hessenberg column describes exactly the vector that is kept
-  const bool use_h2 = have_h2;
-  if (use_h2)
-    for (int i = 0; i <= j; ++i) col[i] = col[i] + kw.h2[i * kw.nrhs + b];
-  const double hn2 = use_h2 ? nn - s2 : nn;
-  const double hn = hn2 > 0.0 ? sqrt(hn2) : 0.0;
-  kw.nrm[b] = hn > 0.0 ? 1.0 / hn : 0.0;
-  if (kw.lazy) {
-    kw.fix[b] = use_h2;
-    kw.vscale[(j + 1) * kw.nrhs + b] = use_h2 ? 1.0 : kw.nrm[b];
-  }
-  col[j + 1] = mk<double>(hn, 0.0);
-  const int K = kw.kmax;
+  const int done = kw.done[b];
+  if (threadIdx.x == 0) skip_before[b] = done;
+  if (done) return;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, n = kw.nrhs, K = kw.kmax;
+  __shared__ cx<double> col[40], h1[40], h2[40], cs[40], sn[40];
+  __shared__ double nns;
   cx<double>* Hb = kw.H + (int64_t)b * (K + 1) * K;
   cx<double>* csb = kw.cs + (int64_t)b * K;
   cx<double>* snb = kw.sn + (int64_t)b * K;
   cx<double>* gb = kw.gv + (int64_t)b * (K + 1);
-  for (int i = 0; i < j; ++i) {
-    const cx<double> a = col[i], c2 = col[i + 1];
-    const cx<double> t = csb[i] * a + snb[i] * c2;
-    col[i + 1] = cmulc(snb[i], a) * mk<double>(-1.0, 0.0) + cmulc(csb[i], c2);
-    col[i] = t;
+  // h2 and ||w'||^2 (lazy mode: h2 exists only where fix[b] was raised)
+  const bool use_h2 = !kw.lazy || kw.fix[b];
+  if (threadIdx.x <= j) {
+    h1[threadIdx.x] = kw.h1[threadIdx.x * n + b];
+    if ((int)threadIdx.x < j) {
+      cs[threadIdx.x] = csb[threadIdx.x];
+      sn[threadIdx.x] = snb[threadIdx.x];
+    }
   }
-  const cx<double> a = col[j], bb = col[j + 1];
+  if (wid == 3) {
+    double nn = 0.0;
+    for (int c = lane; c < kw.nchunk; c += 512) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = c + 64 * u < kw.nchunk ? kw.partn[(int64_t)(c + 64 * u) * n + b] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) nn += v[u];
+    }
+    nn = wave_sum(nn);
+    if (lane == 0) nns = nn;
+  }
+  if (use_h2)
+    for (int i = wid; i <= j; i += 4) {
+      double re, im;
+      chunk_sum(kw, i, b, lane, &re, &im);
+      re = wave_sum(re);
+      im = wave_sum(im);
+      if (lane == 0) h2[i] = mk<double>(re, im);
+    }
+  __syncthreads();
+  if (threadIdx.x != 0) {
+    if (use_h2 && (int)threadIdx.x <= j) kw.h2[threadIdx.x * n + b] = h2[threadIdx.x];
+    return;
+  }
+  double s2 = 0.0;
+  if (use_h2) {
+    kw.h2[b] = h2[0];
+    for (int i = 0; i <= j; ++i) s2 += cabs2(h2[i]);
+  }
+  // the Hessenberg column describes exactly the vector that is kept
+  const double hn2 = use_h2 ? nns - s2 : nns;
+  const double hn = hn2 > 0.0 ? sqrt(hn2) : 0.0;
+  kw.nrm[b] = hn > 0.0 ? 1.0 / hn : 0.0;
+  if (kw.lazy) {
+    kw.fix[b] = use_h2;
+    kw.vscale[(j + 1) * n + b] = use_h2 ? 1.0 : kw.nrm[b];
+  }
+  cx<double> next = use_h2 ? h1[0] + h2[0] : h1[0];  // entry i of the rotated column so far
+  for (int i = 0; i < j; ++i) {
+    const cx<double> a = next, c2 = use_h2 ? h1[i + 1] + h2[i + 1] : h1[i + 1];
+    next = cmulc(sn[i], a) * mk<double>(-1.0, 0.0) + cmulc(cs[i], c2);
+    col[i] = cs[i] * a + sn[i] * c2;
+  }
+  const cx<double> a = next, bb = mk<double>(hn, 0.0);
   const double den = sqrt(cabs2(a) + cabs2(bb));
   cx<double> cj, sj;
   if (den > 0.0) {
@@ -845,9 +896,10 @@ __global__ __launch_bounds__(64) void k_hess_givens(KrylovWork kw, int j, double
   col[j] = mk<double>(den, 0.0);
   for (int i = 0; i <= j; ++i) Hb[i + (int64_t)j * (K + 1)] = col[i];
   const cx<double> g = gb[j];
-  gb[j + 1] = cmulc(sj, g) * mk<double>(-1.0, 0.0);
+  const cx<double> gn = cmulc(sj, g) * mk<double>(-1.0, 0.0);
+  gb[j + 1] = gn;
   gb[j] = cj * g;
-  const double est = sqrt(cabs2(gb[j + 1])) / kw.bnorm[b];
+  const double est = sqrt(cabs2(gn)) / kw.bnorm[b];
   if (den > 0.0) {
     kw.kact[b] = j + 1;
     kw.est[b] = est;
@@ -875,9 +927,18 @@ __global__ __launch_bounds__(256) void k_final(KrylovWork kw, const cx<TV>* __re
   const double s = kw.nrm[b];
   for (int64_t p = p0 + threadIdx.x; p < p1; p += 256) {
     cx<double> wv = cvt<TV, double>(w[base + p]);
+    if constexpr (NV <= 10) {
+      cx<TV> vv[NV];
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
-      if (i <= j) wv = wv - hc[i] * cvt<TV, double>(V[i * stride + base + p]);
+      for (int i = 0; i < NV; ++i) vv[i] = V[min(i, j) * stride + base + p];
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        if (i <= j) wv = wv - hc[i] * cvt<TV, double>(vv[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        if (i <= j) wv = wv - hc[i] * cvt<TV, double>(V[i * stride + base + p]);
+    }
     vout[base + p] = cvt<double, TV>(s * wv);
   }
 }
@@ -1150,8 +1211,7 @@ static void arnoldi_nv(const KrylovWork& w, const cx<TV>* V, cx<double>* wv, int
     hipLaunchKernelGGL(k_fix_flags, dim3(w.nrhs), dim3(64), 0, s, w);
     hipLaunchKernelGGL((k_dots<NV, false, TV>), cgrid(w), dim3(256), 0, s, w, V, (const cx<TV>*)vnext, j, w.fix);
   }
-  hipMemcpyAsync(skip_copy, w.done, sizeof(int) * w.nrhs, hipMemcpyDeviceToDevice, s);
-  hipLaunchKernelGGL(k_hess_givens, dim3(w.nrhs), dim3(64), 0, s, w, j, tol);
+  hipLaunchKernelGGL(k_hess_givens, dim3(w.nrhs), dim3(256), 0, s, w, j, tol, skip_copy);
   if constexpr (std::is_same<TV, double>::value) {
     hipLaunchKernelGGL((k_final<NV, double>), cgrid(w), dim3(256), 0, s, w, V,
                        w.lazy ? (const cx<double>*)vnext : wv, vnext, j, skip_copy);
