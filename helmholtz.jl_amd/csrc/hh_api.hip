@@ -258,11 +258,9 @@ struct hh_solver {
   cx<double>* kpart = nullptr; // K-cycle partial inner products
   // Jac-GMRES smoothing: per-RHS complex128 state shared by the levels
   cx<double>* gm_part = nullptr;
-  cx<double>* gm_hc = nullptr;
   cx<double>* gm_H = nullptr;
   double* gm_sc = nullptr;
   double* gm_beta = nullptr;
-  cx<double>* gm_y = nullptr;
   int* conv_d = nullptr;
   double* n2tmp = nullptr;
   double* res_d = nullptr;
@@ -329,8 +327,8 @@ struct hh_solver {
     }
     dfree(kpart);
     kpart = nullptr;
-    dfree(gm_part); dfree(gm_hc); dfree(gm_H); dfree(gm_sc); dfree(gm_beta); dfree(gm_y);
-    gm_part = gm_hc = gm_H = gm_y = nullptr;
+    dfree(gm_part); dfree(gm_H); dfree(gm_sc); dfree(gm_beta);
+    gm_part = gm_H = nullptr;
     gm_sc = gm_beta = nullptr;
     dfree(V); dfree(Z); dfree(xk); dfree(bk); dfree(wk); dfree(b0);
     V = nullptr; Z = nullptr; xk = bk = wk = nullptr; b0 = nullptr;
@@ -524,11 +522,9 @@ void ensure_work(hh_solver* S, int nrhs) {
       L.gv = dalloc<char>((size_t)L.g.N * nrhs * es * (pl + 1));
     }
     S->gm_part = dalloc<cx<double>>(gm_part_elems(nrhs));
-    S->gm_hc = dalloc<cx<double>>((size_t)(GM_MAX_STEPS + 1) * nrhs);
     S->gm_H = dalloc<cx<double>>((size_t)nrhs * (GM_MAX_STEPS + 1) * GM_MAX_STEPS);
-    S->gm_sc = dalloc<double>(nrhs);
+    S->gm_sc = dalloc<double>((size_t)(GM_MAX_STEPS + 1) * nrhs);
     S->gm_beta = dalloc<double>(nrhs);
-    S->gm_y = dalloc<cx<double>>((size_t)nrhs * GM_MAX_STEPS);
   }
   const int64_t N = S->lv[0].g.N;
   const int K = S->p.inner;
@@ -722,13 +718,10 @@ struct Cycle {
     a.d = (const cx<T>*)L.d;
     a.f = (const cx<T>*)L.f;
     a.V = (cx<T>*)L.gv;
-    a.u = (cx<T>*)L.r;
     a.part = S->gm_part;
-    a.hc = S->gm_hc;
     a.H = S->gm_H;
     a.sc = S->gm_sc;
     a.beta = S->gm_beta;
-    a.y = S->gm_y;
     a.skip = skip;
     gm_smooth<T>(a, steps, st);
   }

@@ -172,4 +172,35 @@ __device__ __forceinline__ void tile_of(const TileMap& m, int& xt, int& yt, int&
   rhs = (int)(L / (unsigned)m.nyt) * m.G + r_in;
 }
 
+// Sums of M values over a wavefront, the values shared out among the lanes as
+// the reduction narrows: at each step a lane keeps one half of its values and
+// hands the other half to its partner, so M = 21 takes 23 exchanges where M
+// separate reductions take 126 (the same tree of additions, the same bits).
+// On return v[0 .. K) holds the sums of values base .. base + valid - 1.
+template <int M, int O>
+struct WaveSums {
+  static constexpr int Hf = (M + 1) / 2;
+  template <typename F>
+  static __device__ __forceinline__ void run(const double (&v)[M], int lane, int base, int valid, F&& put) {
+    double h[Hf];
+    const bool hi = (lane & O) != 0;
+#pragma unroll
+    for (int k = 0; k < Hf; ++k) {
+      const double up = k + Hf < M ? v[k + Hf < M ? k + Hf : 0] : 0.0;
+      const double send = M > 1 && hi ? v[k] : up, keep = M > 1 && hi ? up : v[k];
+      h[k] = keep + __shfl_xor(M > 1 ? send : v[k], O, 64);
+    }
+    if (M > 1) {
+      base = hi ? base + Hf : base;
+      valid = hi ? valid - Hf : min(valid, Hf);
+    }
+    if constexpr (O > 1)
+      WaveSums<Hf, O / 2>::run(h, lane, base, valid, put);
+    else
+#pragma unroll
+      for (int k = 0; k < Hf; ++k)
+        if (k < valid) put(base + k, h[k]);
+  }
+};
+
 }  // namespace hh

@@ -236,10 +236,9 @@ void adjoint_map(const Grid& g, cx<double>* v, int nrhs, int mode, hipStream_t s
 constexpr int GM_MAX_STEPS = 8;  // GMRES steps per smoothing call
 // One level's operands and workspace: b, x (updated in place; zero_x: x = 0
 // on entry and is written), diagonal d and damped-Jacobi factor f, basis V
-// ((GM_MAX_STEPS + 1) blocks of N x nrhs), u (one block), and the per-RHS
-// complex128 state: part (gm_part_elems), hc ((GM_MAX_STEPS + 1) x nrhs),
-// H (nrhs x (GM_MAX_STEPS + 1) x GM_MAX_STEPS), sc, beta (nrhs), y
-// (nrhs x GM_MAX_STEPS).
+// ((GM_MAX_STEPS + 1) blocks of N x nrhs), and the per-RHS complex128 state:
+// part (gm_part_elems), H (nrhs x (GM_MAX_STEPS + 1) x GM_MAX_STEPS), sc
+// ((GM_MAX_STEPS + 1) x nrhs), beta (nrhs).
 template <typename T>
 struct GmArgs {
   Grid g;
@@ -250,13 +249,10 @@ struct GmArgs {
   const cx<T>* d;
   const cx<T>* f;
   cx<T>* V;
-  cx<T>* u;
   cx<double>* part;
-  cx<double>* hc;
   cx<double>* H;
   double* sc;
   double* beta;
-  cx<double>* y;
   const int* skip;
 };
 size_t gm_part_elems(int nrhs);
