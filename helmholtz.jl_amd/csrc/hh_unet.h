@@ -38,8 +38,8 @@ struct UNet {
   // parameters (device, fp32 master + bf16 copies)
   float* w[UNET_NCONV] = {};      // [9][co][ci]
   float* b[UNET_NCONV] = {};      // [co]
-  bf16* wb[UNET_NCONV] = {};      // forward copy [9][co][ci]
-  bf16* wt[UNET_NCONV] = {};      // backward-data copy [9][ci][co], taps flipped
+  bf16* wb[UNET_NCONV] = {};      // forward copy, MFMA operand order (k_wcopy)
+  bf16* wt[UNET_NCONV] = {};      // backward-data copy, taps flipped
   float* hw = nullptr;            // head 1x1: [2][16]
   float* hb = nullptr;            // [2]
   float* flat = nullptr;          // all parameters, contiguous (w, b per layer, then head)

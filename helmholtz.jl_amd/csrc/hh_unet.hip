@@ -5,10 +5,8 @@
 // Layout: activations NHWC with the pixel index x-fastest (p = i + nx*j, the
 // solver's nodal order) and channels contiguous (multiples of 16).
 // 3x3 convolution = implicit GEMM: out[p][co] = sum_{tap,ci} W[tap][co][ci]
-// in[p + off(tap)][ci] (zero padding).  One wavefront computes 16 pixels x all
-// output channels (the A operand, 16 pixels x 16 input channels, is loaded once
-// and reused for every 16-channel output block).  Backward-data is the same
-// kernel on the output gradient with W transposed and taps flipped; the
+// in[p + off(tap)][ci] (zero padding), a tile of pixels per block with its inputs
+// in LDS.  Backward-data is the same kernel on the output gradient with W transposed and taps flipped; the
 // weight gradient is a split-K MFMA over pixels with per-chunk partials summed
 // in a fixed order (deterministic).  Down-sampling is nodal full weighting
 // ([1 2 1]/4 per axis, stride 2, zero padding) and up-sampling nodal
@@ -63,77 +61,150 @@ static T* dmal(size_t n) {
 }
 
 // ------------------------------------------------------------------ kernels
-// A wavefront computes PM x 16 pixels x NCO * 16 output channels (channel
-// block blockIdx.z of a layer with `cout` outputs).  Every operand load of a
-// (tap, 16-channel) step feeds several MFMAs: the input tile of a pixel group
-// is used for the NCO channel blocks, the weight tile for the PM pixel groups
-// (with one of each, two 512-byte loads per MFMA kept the loads, not the
-// matrix cores, busy).  NCO and PM are picked per launch so that small grids
-// still give several wavefronts per SIMD.
-template <int NCO, int PM>
-__global__ __launch_bounds__(256) void k_conv3x3(const bf16* __restrict__ in, int cin, const bf16* __restrict__ w,
-                                                 const float* __restrict__ bias, bf16* __restrict__ out, int nx,
-                                                 int ny, int relu, int cout) {
-  const int img = blockIdx.y;
-  const int npix = nx * ny;
+// The channels of an activation: [0, ca) in a, [ca, ca + cb) in b (the up-sampled
+// and the skip part of a decoder layer's input; b is unused for one block)
+struct Src {
+  const bf16* a;
+  const bf16* b;
+  int ca, cb;
+};
+struct Dst {
+  bf16* a;
+  bf16* b;
+  int ca, cb;
+};
+
+// A block computes a tile of tw x th pixels x wc NCO 16 output channels (channel
+// block blockIdx.z): its four wavefronts are 4 / wc groups of pixels (G times the
+// 16 pixels of an MFMA operand each, counted along the tile's rows) times wc
+// groups of NCO channel blocks.  The tile's inputs with their one-pixel ring, all
+// channels, are staged in LDS once (16-byte loads, zero outside the image; 16
+// bytes of padding per pixel: the 16 pixels of an operand hit distinct banks), so
+// that the nine taps read LDS.  The weights come in operand order (512 contiguous
+// bytes per operand) and three (tap, 16-channel) steps ahead.  With the weights as
+// the MFMA's rows a lane ends with four channels of one pixel: 8-byte stores.  A
+// gradient leaves with the producing layer's ReLU mask applied where `mask` is
+// that layer's output.
+// The products' order (taps, then channel blocks, one accumulator per output) is
+// that of the kernel before, which loaded pixels nine times over from L1 with a
+// bounds test each and masked, joined and split activations in passes of their
+// own.  One loss and gradient for 16 images of 129 x 129 on MI355X: the 27
+// convolutions 690 us and those passes 197 us there, 325 us here in all, 125 TFLOP/s:
+// the level-0 layers are bound by activations (12 us a
+// launch against 4 us at the copy rate), the small levels by the chain of LDS
+// reads and products of their one or two wavefronts per SIMD.
+template <int NCO, int G>
+__global__ __launch_bounds__(256) void k_conv3x3(Src in, const bf16* __restrict__ w, const float* __restrict__ bias,
+                                                 Dst out, const bf16* __restrict__ mask, int nx, int ny, int relu,
+                                                 int wc, int tw, int th, int xtiles) {
+  extern __shared__ __align__(16) bf16 tile[];
+  __shared__ int pix[256];
+  const int cin = in.ca + in.cb, nb = (out.ca + out.cb) / 16;
+  const int64_t ipx = (int64_t)blockIdx.y * nx * ny;  // the image's first pixel
+  const int x0 = (int)(blockIdx.x % (unsigned)xtiles) * tw, y0 = (int)(blockIdx.x / (unsigned)xtiles) * th;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int tile = (blockIdx.x * 4 + wv) * 16 * PM;
-  if (tile >= npix) return;  // uniform per wavefront
-  const int co0 = blockIdx.z * NCO * 16;
-  const int m = lane & 15;
-  const int kq = (lane >> 4) * 4;
-  int ia[PM], ja[PM];
-  bool pa_ok[PM];
-#pragma unroll
-  for (int g = 0; g < PM; ++g) {
-    const int pa = tile + 16 * g + m;
-    pa_ok[g] = pa < npix;
-    ia[g] = pa_ok[g] ? pa % nx : 0;
-    ja[g] = pa_ok[g] ? pa / nx : 0;
+  const int m = lane & 15, kq = (lane >> 4) * 4;
+  const int cob0 = ((int)blockIdx.z * wc + wv % wc) * NCO, grp0 = (wv / wc) * G;
+  const int ld = cin + 8, nch = cin / 8, sw = tw + 2;
+  // output pixel of each of the tile's pixels (-1: none)
+  if ((int)threadIdx.x < 64 * G / wc) {
+    const int ly = (int)threadIdx.x / tw, lx = (int)threadIdx.x - ly * tw;
+    pix[threadIdx.x] = ly < th && x0 + lx < nx && y0 + ly < ny ? (y0 + ly) * nx + x0 + lx : -1;
   }
-  const bf16* inb = in + (int64_t)img * npix * cin;
-  f4 acc[PM][NCO];
+  const int items = sw * (th + 2) * nch;
+  for (int e0 = threadIdx.x; e0 < items; e0 += 1024) {
+    uint4 v[4];
+    int d[4];
 #pragma unroll
-  for (int g = 0; g < PM; ++g)
+    for (int u = 0; u < 4; ++u) {
+      const int e = e0 + 256 * u;
+      const int px = e / nch, ch = (e - px * nch) * 8, ly = px / sw, lx = px - ly * sw;
+      const int gx = x0 - 1 + lx, gy = y0 - 1 + ly;
+      d[u] = e < items ? px * ld + ch : -1;
+      v[u] = make_uint4(0u, 0u, 0u, 0u);
+      if (e < items && gx >= 0 && gx < nx && gy >= 0 && gy < ny) {
+        const int64_t q = ipx + (int64_t)gy * nx + gx;
+        v[u] = *(const uint4*)(ch < in.ca ? in.a + q * in.ca + ch : in.b + q * in.cb + (ch - in.ca));
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (d[u] >= 0) *(uint4*)(tile + d[u]) = v[u];
+  }
+  f4 acc[G][NCO];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int c = 0; c < NCO; ++c) acc[g][c] = f4{0.f, 0.f, 0.f, 0.f};
-  for (int tap = 0; tap < 9; ++tap) {
-    const bf16* src[PM];
-    bool ok[PM];
+  const int steps = 9 * (cin / 16);
+  const bf16* wl = w + ((int64_t)cob0 * 64 + lane) * 4;
+  const int64_t wstep = (int64_t)nb * 256;
+  s4 a[3][NCO];
 #pragma unroll
-    for (int g = 0; g < PM; ++g) {
-      const int ii = ia[g] + tap % 3 - 1, jj = ja[g] + tap / 3 - 1;
-      ok[g] = pa_ok[g] && ii >= 0 && ii < nx && jj >= 0 && jj < ny;
-      src[g] = inb + ((int64_t)(ok[g] ? jj : 0) * nx + (ok[g] ? ii : 0)) * cin + kq;
-    }
-    const bf16* wtap = w + (int64_t)tap * cout * cin + (int64_t)(co0 + m) * cin + kq;
-    for (int cb = 0; cb < cin; cb += 16) {
-      s4 a[PM];
+  for (int u = 0; u < 3; ++u)
 #pragma unroll
-      for (int g = 0; g < PM; ++g) a[g] = ok[g] ? *(const s4*)(src[g] + cb) : s4{0, 0, 0, 0};
+    for (int c = 0; c < NCO; ++c) a[u][c] = *(const s4*)(wl + u * wstep + c * 256);
+  const bf16* tl[G];
 #pragma unroll
-      for (int c = 0; c < NCO; ++c) {
-        const s4 bv = *(const s4*)(wtap + (int64_t)c * 16 * cin + cb);
+  for (int g = 0; g < G; ++g) {
+    const int p = (grp0 + g) * 16 + m, ly = p / tw;
+    tl[g] = tile + (ly < th ? ly * sw + p - ly * tw : 0) * ld + kq;
+  }
+  __syncthreads();
+  int cb = 0, dx = 0, row = 0;
+  for (int s = 0; s < steps; s += 3) {
 #pragma unroll
-        for (int g = 0; g < PM; ++g) acc[g][c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[g], bv, acc[g][c], 0, 0, 0);
+    for (int u = 0; u < 3; ++u) {
+      const int o = row + dx * ld + cb;
+      s4 b[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) b[g] = *(const s4*)(tl[g] + o);
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int c = 0; c < NCO; ++c)
+          acc[g][c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[u][c], b[g], acc[g][c], 0, 0, 0);
+      // (the last steps load their own operands again)
+      const int nx3 = s + u + 3 < steps ? s + u + 3 : s + u;
+#pragma unroll
+      for (int c = 0; c < NCO; ++c) a[u][c] = *(const s4*)(wl + nx3 * wstep + c * 256);
+      cb += 16;
+      if (cb == cin) {
+        cb = 0;
+        if (++dx == 3) {
+          dx = 0;
+          row += sw * ld;
+        }
       }
     }
   }
-  bf16* ob = out + (int64_t)img * npix * cout;
 #pragma unroll
-  for (int g = 0; g < PM; ++g)
+  for (int c = 0; c < NCO; ++c) {
+    const int co = (cob0 + c) * 16 + kq;
+    const bool first = co < out.ca;
+    bf16* ob = first ? out.a + co : out.b + (co - out.ca);
+    const int st = first ? out.ca : out.cb;
+    const float4 bi = bias ? *(const float4*)(bias + co) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int c = 0; c < NCO; ++c)
+    for (int g = 0; g < G; ++g) {
+      const int p = pix[(grp0 + g) * 16 + m];
+      if (p < 0) continue;
+      float v[4] = {acc[g][c][0] + bi.x, acc[g][c][1] + bi.y, acc[g][c][2] + bi.z, acc[g][c][3] + bi.w};
+      s4 r;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int p = tile + 16 * g + kq + i;
-        const int co = co0 + c * 16 + m;
-        if (p < npix) {
-          float v = acc[g][c][i] + (bias ? bias[co] : 0.f);
-          if (relu) v = v > 0.f ? v : 0.f;
-          ob[(int64_t)p * cout + co] = f2bf(v);
-        }
+        if (relu) v[i] = v[i] > 0.f ? v[i] : 0.f;
+        r[i] = (short)f2bf(v[i]);
       }
+      const int64_t q = (ipx + p) * st;
+      if (mask) {
+        const s4 y = *(const s4*)(mask + q + co);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = bf2f((bf16)y[i]) > 0.f ? r[i] : (short)0;
+      }
+      *(s4*)(ob + q) = r;
+    }
+  }
 }
 
 // Weight and bias gradients of a 3x3 layer as one MFMA GEMM per tap over
@@ -172,16 +243,17 @@ __device__ __forceinline__ void store_px4(bf16* dst, const uint4 (&v)[4]) {
   }
 }
 template <int NCO>
-__global__ __launch_bounds__(256) void k_conv_wgrad(const bf16* __restrict__ dpre, const bf16* __restrict__ in,
-                                                   int cin, int nx, int ny, int64_t total, int64_t per,
-                                                   float* __restrict__ part) {
+__global__ __launch_bounds__(256) void k_conv_wgrad(const bf16* __restrict__ dpre, Src src, int nx, int ny,
+                                                   int64_t total, int64_t per, float* __restrict__ part) {
   constexpr int COUT = 16 * NCO;
   constexpr int NTILE = 9 * NCO;
   constexpr int TPW = (NTILE + 3) / 4;
   __shared__ __align__(16) bf16 sA[COUT * WG_LD];
   __shared__ __align__(16) bf16 sB[9 * 16 * WG_LD];
   __shared__ int sbase[WG_PX], si[WG_PX], sj[WG_PX];
-  const int cib = blockIdx.y;
+  const int cib = blockIdx.y, cin = src.ca + src.cb;
+  const bf16* __restrict__ in = cib * 16 < src.ca ? src.a + cib * 16 : src.b + (cib * 16 - src.ca);
+  const int ild = cib * 16 < src.ca ? src.ca : src.cb;  // the block's 16 channels at in + pixel ild
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int m = lane & 15, kq = (lane >> 4) * 4;
   const int npix = nx * ny;
@@ -231,7 +303,7 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const bf16* __restrict__ dpr
         if (img >= 0) {
           const int ii = si[px] + t % 3 - 1, jj = sj[px] + t / 3 - 1;
           if (ii >= 0 && ii < nx && jj >= 0 && jj < ny)
-            v[i] = *(const uint4*)(in + ((int64_t)img * npix + (int64_t)jj * nx + ii) * cin + cib * 16 + c8);
+            v[i] = *(const uint4*)(in + ((int64_t)img * npix + (int64_t)jj * nx + ii) * ild + c8);
         }
       }
       store_px4(sB + (t * 16 + c8) * WG_LD + 4 * px4, v);
@@ -294,96 +366,111 @@ __global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ par
   }
 }
 
-__global__ __launch_bounds__(256) void k_relu_bwd(const bf16* __restrict__ dout, const bf16* __restrict__ out,
-                                                  bf16* __restrict__ dpre, int64_t n) {
-  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (k < n) dpre[k] = bf2f(out[k]) > 0.f ? dout[k] : (bf16)0;
+// Eight channels of a pixel as floats, and back (rounded)
+__device__ __forceinline__ void ld8(const bf16* p, float (&v)[8]) {
+  const uint4 u = *(const uint4*)p;
+  const unsigned w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    v[2 * h] = __builtin_bit_cast(float, w[h] << 16);
+    v[2 * h + 1] = __builtin_bit_cast(float, w[h] & 0xffff0000u);
+  }
+}
+__device__ __forceinline__ void st8(bf16* p, const float (&v)[8], const bf16* __restrict__ mask) {
+  float y[8];
+  if (mask) ld8(mask, y);
+  unsigned w[4];
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    const unsigned lo = !mask || y[2 * h] > 0.f ? f2bf(v[2 * h]) : 0u;
+    const unsigned hi = !mask || y[2 * h + 1] > 0.f ? f2bf(v[2 * h + 1]) : 0u;
+    w[h] = lo | (hi << 16);
+  }
+  *(uint4*)p = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// nodal full weighting, stride 2, zero padding; out = scale * R in
+// Nodal full weighting, stride 2, zero padding: out = scale * R in, with the ReLU
+// mask of `mask` (that layer's output, or null).  A thread takes eight channels of
+// a pixel (16-byte accesses, one index decomposition for the eight: the training
+// batch's six launches 36 us, one value per thread 60 us; k_up's 38 and 127 us);
+// blockIdx.y is the image.
 __global__ __launch_bounds__(256) void k_down(const bf16* __restrict__ in, int C, int nx, int ny, bf16* __restrict__ out,
-                                              int ncx, int ncy, int nimg, float scale) {
-  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t nc = (int64_t)ncx * ncy;
-  if (k >= nc * nimg * C) return;
-  const int c = (int)(k % C);
-  const int64_t q = k / C;
-  const int64_t img = q / nc;
-  const int pc = (int)(q - img * nc);
-  const int I = pc % ncx, J = pc / ncx;
+                                              int ncx, int ncy, float scale, const bf16* __restrict__ mask) {
+  const unsigned k = blockIdx.x * 256 + threadIdx.x;
+  const unsigned c8 = C / 8, nc = (unsigned)ncx * ncy, q = k / c8;
+  if (q >= nc) return;
+  const int c = (int)(k - q * c8) * 8;
+  const int J = (int)(q / (unsigned)ncx), I = (int)q - J * ncx;
+  const bf16* ib = in + (int64_t)blockIdx.y * nx * ny * C + c;
   const float wgt[3] = {0.25f, 0.5f, 0.25f};
-  float s = 0.f;
+  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
   for (int b = -1; b <= 1; ++b) {
     const int j = 2 * J + b;
     if (j < 0 || j >= ny) continue;
+#pragma unroll
     for (int a = -1; a <= 1; ++a) {
       const int i = 2 * I + a;
       if (i < 0 || i >= nx) continue;
-      s += wgt[a + 1] * wgt[b + 1] * bf2f(in[((img * ny + j) * (int64_t)nx + i) * C + c]);
+      float v[8];
+      ld8(ib + ((int64_t)j * nx + i) * C, v);
+#pragma unroll
+      for (int h = 0; h < 8; ++h) s[h] += wgt[a + 1] * wgt[b + 1] * v[h];
     }
   }
-  out[k] = f2bf(scale * s);
+#pragma unroll
+  for (int h = 0; h < 8; ++h) s[h] *= scale;
+  const int64_t o = ((int64_t)blockIdx.y * nc + q) * C + c;
+  st8(out + o, s, mask ? mask + o : nullptr);
 }
 
-// nodal bilinear prolongation; out (+)= scale * P in
+// Nodal bilinear prolongation: out (+)= scale * P in, masked and split over threads
+// as k_down
 __global__ __launch_bounds__(256) void k_up(const bf16* __restrict__ in, int C, int ncx, int ncy, bf16* __restrict__ out,
-                                            int nx, int ny, int nimg, float scale, int accumulate) {
-  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t nf = (int64_t)nx * ny;
-  if (k >= nf * nimg * C) return;
-  const int c = (int)(k % C);
-  const int64_t q = k / C;
-  const int64_t img = q / nf;
-  const int p = (int)(q - img * nf);
-  const int i = p % nx, j = p / nx;
+                                            int nx, int ny, float scale, int accumulate,
+                                            const bf16* __restrict__ mask) {
+  const unsigned k = blockIdx.x * 256 + threadIdx.x;
+  const unsigned c8 = C / 8, nf = (unsigned)nx * ny, q = k / c8;
+  if (q >= nf) return;
+  const int c = (int)(k - q * c8) * 8;
+  const int j = (int)(q / (unsigned)nx), i = (int)q - j * nx;
   const int i0 = i >> 1, j0 = j >> 1;
-  const int i1 = (i & 1) ? i0 + 1 : i0, j1 = (j & 1) ? j0 + 1 : j0;
-  const float wi = (i & 1) ? 0.5f : 1.f, wj = (j & 1) ? 0.5f : 1.f;
-  auto at = [&](int a, int b) {
-    return (a < ncx && b < ncy) ? bf2f(in[((img * ncy + b) * (int64_t)ncx + a) * C + c]) : 0.f;
+  const bf16* ib = in + (int64_t)blockIdx.y * ncx * ncy * C + c;
+  auto at = [&](int a, int b, float (&v)[8]) {
+    if (a < ncx && b < ncy) {
+      ld8(ib + ((int64_t)b * ncx + a) * C, v);
+    } else {
+#pragma unroll
+      for (int h = 0; h < 8; ++h) v[h] = 0.f;
+    }
   };
-  float s;
-  if ((i & 1) && (j & 1))
-    s = 0.25f * (at(i0, j0) + at(i1, j0) + at(i0, j1) + at(i1, j1));
-  else if (i & 1)
-    s = 0.5f * (at(i0, j0) + at(i1, j0));
-  else if (j & 1)
-    s = 0.5f * (at(i0, j0) + at(i0, j1));
-  else
-    s = at(i0, j0);
-  (void)wi;
-  (void)wj;
-  s *= scale;
-  if (accumulate) s += bf2f(out[k]);
-  out[k] = f2bf(s);
-}
-
-__global__ __launch_bounds__(256) void k_concat(const bf16* __restrict__ a, int Ca, const bf16* __restrict__ b, int Cb,
-                                                bf16* __restrict__ out, int64_t npix) {
-  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int C = Ca + Cb;
-  if (k >= npix * C) return;
-  const int c = (int)(k % C);
-  const int64_t p = k / C;
-  out[k] = c < Ca ? a[p * Ca + c] : b[p * Cb + (c - Ca)];
-}
-
-// da = dc[:, :Ca] ; db += dc[:, Ca:]
-__global__ __launch_bounds__(256) void k_split(const bf16* __restrict__ dc, int Ca, int Cb, bf16* __restrict__ da,
-                                               bf16* __restrict__ db, int accumulate_b, int64_t npix) {
-  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int C = Ca + Cb;
-  if (k >= npix * C) return;
-  const int c = (int)(k % C);
-  const int64_t p = k / C;
-  if (c < Ca) {
-    da[p * Ca + c] = dc[k];
-  } else {
-    const int64_t o = p * Cb + (c - Ca);
-    float v = bf2f(dc[k]);
-    if (accumulate_b) v += bf2f(db[o]);
-    db[o] = f2bf(v);
+  float s[8], v[8];
+  at(i0, j0, s);
+  if (i & 1) {
+    at(i0 + 1, j0, v);
+#pragma unroll
+    for (int h = 0; h < 8; ++h) s[h] += v[h];
   }
+  if (j & 1) {
+    at(i0, j0 + 1, v);
+#pragma unroll
+    for (int h = 0; h < 8; ++h) s[h] += v[h];
+    if (i & 1) {
+      at(i0 + 1, j0 + 1, v);
+#pragma unroll
+      for (int h = 0; h < 8; ++h) s[h] += v[h];
+    }
+  }
+  const float f = ((i & 1) ? 0.5f : 1.f) * ((j & 1) ? 0.5f : 1.f);
+  const int64_t o = ((int64_t)blockIdx.y * nf + q) * C + c;
+#pragma unroll
+  for (int h = 0; h < 8; ++h) s[h] = f * s[h] * scale;
+  if (accumulate) {
+    ld8(out + o, v);
+#pragma unroll
+    for (int h = 0; h < 8; ++h) s[h] += v[h];
+  }
+  st8(out + o, s, mask ? mask + o : nullptr);
 }
 
 // 1x1 head: y[p][o] = hb[o] + sum_c hw[o][c] x[p][c], 16 -> 2, fp32 out
@@ -402,7 +489,7 @@ __global__ __launch_bounds__(256) void k_head_fwd(const bf16* __restrict__ x, co
   y[2 * p + 1] = y1;
 }
 
-// dx = hw^T dy (bf16); per-block partial sums of dhw (2x16) and dhb (2)
+// dx = hw^T dy (bf16) with x's own ReLU mask (x is a layer's output); per-block partial sums of dhw (2x16) and dhb (2)
 __global__ __launch_bounds__(256) void k_head_bwd(const bf16* __restrict__ x, const float* __restrict__ hw,
                                                   const float* __restrict__ dy, bf16* __restrict__ dx, int64_t npix,
                                                   int64_t chunk, float* __restrict__ part) {
@@ -419,7 +506,7 @@ __global__ __launch_bounds__(256) void k_head_bwd(const bf16* __restrict__ x, co
       const float v = bf2f(x[p * 16 + c]);
       acc[c] += d0 * v;
       acc[16 + c] += d1 * v;
-      dx[p * 16 + c] = f2bf(hw[c] * d0 + hw[16 + c] * d1);
+      dx[p * 16 + c] = v > 0.f ? f2bf(hw[c] * d0 + hw[16 + c] * d1) : (bf16)0;
     }
     acc[32] += d0;
     acc[33] += d1;
@@ -467,7 +554,9 @@ __global__ __launch_bounds__(256) void k_adam(float* __restrict__ w, const float
   w[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + eps);
 }
 
-// wb[tap][co][ci] = bf16(w[tap][co][ci]); wt[tap][ci][co] = bf16(w[8 - tap][co][ci])
+// bf16 copies in operand order: 16 x 16 blocks [tap][k / 16][m / 16] of 64 lanes x 4
+// values, lane (m % 16) + 16 ((k % 16) / 4), value k % 4.  wb: m = co, k = ci; wt:
+// m = ci, k = co, taps flipped.
 __global__ __launch_bounds__(256) void k_wcopy(const float* __restrict__ w, bf16* __restrict__ wb, bf16* __restrict__ wt,
                                                int co, int ci) {
   const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -477,9 +566,12 @@ __global__ __launch_bounds__(256) void k_wcopy(const float* __restrict__ w, bf16
   const int64_t r = k / ci;
   const int c_o = (int)(r % co);
   const int tap = (int)(r / co);
+  auto at = [](int t, int kk, int nk, int m, int nm) {
+    return ((((int64_t)t * (nk / 16) + kk / 16) * (nm / 16) + m / 16) * 64 + m % 16 + 16 * (kk % 16 / 4)) * 4 + kk % 4;
+  };
   const bf16 v = f2bf(w[k]);
-  wb[k] = v;
-  wt[((int64_t)(8 - tap) * ci + c_i) * co + c_o] = v;
+  wb[at(tap, c_i, ci, c_o, co)] = v;
+  wt[at(8 - tap, c_o, co, c_i, ci)] = v;
 }
 
 __device__ __forceinline__ uint64_t mix64(uint64_t x) {
@@ -590,22 +682,23 @@ void UNetWork::release() {
   nimg = nx = ny = 0;
 }
 
-// buffers: [0, A_NUM) activations, [A_NUM, 2 A_NUM) gradients, then dpre and
-// d(head input).  Reallocated when the shape grows; a smaller batch of the same
-// grid reuses them (launches index with their own nimg).
+// buffers: [0, A_NUM) activations, [A_NUM, 2 A_NUM) gradients (none for the decoder
+// inputs A_C*, which are read and written as their two parts).  Reallocated when
+// the shape grows; a smaller batch of the same grid reuses them (launches index
+// with their own nimg).
+static bool is_joined(int a) { return a == A_C0 || a == A_C1 || a == A_C2; }
 static void ensure_ws(UNetWork& ws, int nimg, int nx, int ny) {
   if (ws.nx == nx && ws.ny == ny && nimg <= ws.nimg && !ws.bufs.empty()) return;
   for (void* p : ws.bufs)
     if (p) (void)hipFree(p);
-  ws.bufs.assign(2 * A_NUM + 2, nullptr);
+  ws.bufs.assign(2 * A_NUM, nullptr);
   ws.nimg = ws.nx = ws.ny = 0;
   Dims d = dims_of(nimg, nx, ny);
   for (int a = 0; a < A_NUM; ++a) {
+    if (is_joined(a)) continue;
     ws.bufs[a] = dmal<bf16>((size_t)d.T[kActLevel[a]] * kActC[a]);
     ws.bufs[A_NUM + a] = dmal<bf16>((size_t)d.T[kActLevel[a]] * kActC[a]);
   }
-  ws.bufs[2 * A_NUM] = dmal<bf16>((size_t)d.T[0] * 64);      // dpre scratch
-  ws.bufs[2 * A_NUM + 1] = dmal<bf16>((size_t)d.T[0] * 16);  // d(head input)
   ws.nimg = nimg;
   ws.nx = nx;
   ws.ny = ny;
@@ -614,60 +707,123 @@ static void ensure_ws(UNetWork& ws, int nimg, int nx, int ny) {
 static bf16* act(UNetWork& ws, int a) { return (bf16*)ws.bufs[a]; }
 static bf16* grd(UNetWork& ws, int a) { return (bf16*)ws.bufs[A_NUM + a]; }
 
-// output channels (NCO 16-channel blocks) and pixel groups (PM groups of 16)
-// per wavefront: the fewest operand loads per MFMA (1 / NCO + 1 / PM) with
-// NCO * PM <= 8 (at most 32 accumulator registers: six or more wavefronts per
-// SIMD) that still leaves 2048 wavefronts (two per SIMD)
-static void conv_shape(int cout, int64_t pixels, int* nco_out, int* pm_out) {
-  const int nb = cout / 16;
-  const int64_t groups = (pixels + 15) / 16;
-  int best_nco = 1, best_pm = 1;
-  double best = 2.0;
-  for (int nco : {8, 6, 4, 3, 2, 1}) {
-    if (nb % nco) continue;
-    for (int pm : {4, 2, 1}) {
-      if (nco * pm > 8) continue;
-      const int64_t waves = (groups + pm - 1) / pm * (nb / nco);
-      const double loads = 1.0 / nco + 1.0 / pm;
-      if (waves >= 2048 && loads < best - 1e-9) {
-        best = loads;
-        best_nco = nco;
-        best_pm = pm;
-      }
+// the two parts of a decoder layer's input: up-sampled, skip
+static void parts_of(int a, int* up, int* skip) {
+  *up = a == A_C0 ? A_U0 : a == A_C1 ? A_U1 : A_U2;
+  *skip = a == A_C0 ? A_S0 : a == A_C1 ? A_S1 : A_S2;
+}
+static Src src_of(UNetWork& ws, int a, const bf16* x) {
+  if (a < 0) return {x, nullptr, UNET_CIN, 0};
+  if (!is_joined(a)) return {act(ws, a), nullptr, kActC[a], 0};
+  int u, k;
+  parts_of(a, &u, &k);
+  return {act(ws, u), act(ws, k), kActC[u], kActC[k]};
+}
+static Dst grad_of(UNetWork& ws, int a) {
+  if (!is_joined(a)) return {grd(ws, a), nullptr, kActC[a], 0};
+  int u, k;
+  parts_of(a, &u, &k);
+  return {grd(ws, u), grd(ws, k), kActC[u], kActC[k]};
+}
+static bool is_conv_out(int a) {
+  for (int o : kOut)
+    if (o == a) return true;
+  return false;
+}
+
+// Shape of a convolution launch: G pixel groups and NCO channel blocks per
+// wavefront, wc channel groups per block, tiles of tw x th pixels
+struct ConvShape {
+  int nco, g, wc, tw, th, xt, yt;
+  size_t lds;
+};
+constexpr size_t CONV_LDS = 63 << 10;  // the largest tile (64 KiB less the pixel table)
+// Tile of at most P pixels: the width (the image's, split evenly) for which the
+// MFMAs, work done for the tile's unused slots included, and the staged pixels
+// come to the least; false if no tile fits the LDS
+static bool conv_tile(ConvShape* c, int P, int cin, int nx, int ny) {
+  double best = 0;
+  c->lds = 0;
+  for (int w = 4; w <= 32; ++w) {
+    const int xt = (nx + w - 1) / w, tw = (nx + xt - 1) / xt;
+    int th = P / tw < ny ? P / tw : ny;
+    if (th < 1) continue;
+    const int yt = (ny + th - 1) / th;
+    th = (ny + yt - 1) / yt;
+    const int staged = (tw + 2) * (th + 2);
+    const size_t lds = sizeof(bf16) * staged * (size_t)(cin + 8);
+    const double cost = (double)xt * yt * (2 * P + staged);
+    if (lds <= CONV_LDS && (c->lds == 0 || cost < best)) {
+      best = cost;
+      c->tw = tw;
+      c->th = th;
+      c->xt = xt;
+      c->yt = yt;
+      c->lds = lds;
     }
   }
-  *nco_out = best_nco;
-  *pm_out = best_pm;
+  return c->lds != 0;
+}
+// The fewest operand loads per MFMA (1 / NCO + 1 / G) that still leave 2048
+// wavefronts (two per SIMD), or the most wavefronts.  Channel groups share a
+// block's tile as long as it keeps 64 pixels.
+static ConvShape conv_shape(int cin, int cout, int nimg, int nx, int ny) {
+  const int nb = cout / 16;
+  ConvShape best{};
+  double load = 0;
+  for (int nco : {4, 3, 2, 1})
+    for (int g : {4, 2, 1}) {
+      if (nb % nco) continue;
+      ConvShape c{};
+      c.nco = nco;
+      c.g = g;
+      c.wc = g;
+      while (nb / nco % c.wc) c.wc /= 2;
+      if (!conv_tile(&c, 64 * g / c.wc, cin, nx, ny)) continue;
+      const double waves = 4.0 * c.xt * c.yt * nimg * (nb / (nco * c.wc));
+      const double l = 1.0 / nco + 1.0 / g;
+      if (best.nco == 0 || (waves >= 2048 ? l < load - 1e-9 : load > 2.0)) {
+        best = c;
+        load = waves >= 2048 ? l : 3.0;
+      }
+    }
+  return best;
 }
 
-template <int NCO>
-static void conv_launch_pm(int pm, dim3 gridbase, int npix, const bf16* in, int cin, const bf16* w,
-                           const float* bias, bf16* out, int cout, int nx, int ny, int relu, hipStream_t s) {
-  dim3 grid((unsigned)((npix + 64 * pm - 1) / (64 * pm)), gridbase.y, gridbase.z);
-  switch (pm) {
-    case 1: hipLaunchKernelGGL((k_conv3x3<NCO, 1>), grid, dim3(256), 0, s, in, cin, w, bias, out, nx, ny, relu, cout); break;
-    case 2: hipLaunchKernelGGL((k_conv3x3<NCO, 2>), grid, dim3(256), 0, s, in, cin, w, bias, out, nx, ny, relu, cout); break;
-    case 4: hipLaunchKernelGGL((k_conv3x3<NCO, 4>), grid, dim3(256), 0, s, in, cin, w, bias, out, nx, ny, relu, cout); break;
-    default: throw std::runtime_error("unsupported pixel grouping");
-  }
-}
-
-static void conv_launch(const bf16* in, int cin, const bf16* w, const float* bias, bf16* out, int cout, int nimg, int nx,
-                        int ny, int relu, hipStream_t s) {
-  if (cout % 16 || cin % 16 || cin <= 0) throw std::runtime_error("unsupported channel count");
-  int nco, pm;
-  conv_shape(cout, (int64_t)nimg * nx * ny, &nco, &pm);
-  const dim3 gb(1, nimg, (unsigned)(cout / 16 / nco));
-  const int npix = nx * ny;
-  switch (nco) {
-    case 1: conv_launch_pm<1>(pm, gb, npix, in, cin, w, bias, out, cout, nx, ny, relu, s); break;
-    case 2: conv_launch_pm<2>(pm, gb, npix, in, cin, w, bias, out, cout, nx, ny, relu, s); break;
-    case 3: conv_launch_pm<3>(pm, gb, npix, in, cin, w, bias, out, cout, nx, ny, relu, s); break;
-    case 4: conv_launch_pm<4>(pm, gb, npix, in, cin, w, bias, out, cout, nx, ny, relu, s); break;
-    case 6: conv_launch_pm<6>(pm, gb, npix, in, cin, w, bias, out, cout, nx, ny, relu, s); break;
-    case 8: conv_launch_pm<8>(pm, gb, npix, in, cin, w, bias, out, cout, nx, ny, relu, s); break;
+static void conv_launch(Src in, const bf16* w, const float* bias, Dst out, const bf16* mask, int nimg, int nx, int ny,
+                        int relu, hipStream_t s) {
+  const int cin = in.ca + in.cb, cout = out.ca + out.cb;
+  if (in.ca % 16 || in.cb % 16 || out.ca % 16 || out.cb % 16 || cin <= 0 || cout <= 0)
+    throw std::runtime_error("unsupported channel count");
+  const ConvShape c = conv_shape(cin, cout, nimg, nx, ny);
+  const dim3 grid((unsigned)(c.xt * c.yt), (unsigned)nimg, (unsigned)(cout / 16 / (c.nco * c.wc)));
+#define HH_CONV(N, G)                                                                                                  \
+  case 8 * N + G:                                                                                                      \
+    hipLaunchKernelGGL((k_conv3x3<N, G>), grid, dim3(256), c.lds, s, in, w, bias, out, mask, nx, ny, relu, c.wc, c.tw, \
+                       c.th, c.xt);                                                                                    \
+    break;
+  switch (8 * c.nco + c.g) {
+    HH_CONV(1, 1) HH_CONV(1, 2) HH_CONV(1, 4)
+    HH_CONV(2, 1) HH_CONV(2, 2) HH_CONV(2, 4)
+    HH_CONV(3, 1) HH_CONV(3, 2) HH_CONV(3, 4)
+    HH_CONV(4, 1) HH_CONV(4, 2) HH_CONV(4, 4)
     default: throw std::runtime_error("unsupported channel count");
   }
+#undef HH_CONV
+}
+
+// R and P between level lf and lf + 1 (k_down, k_up)
+static void down_launch(const Dims& d, int nimg, const bf16* in, bf16* out, int C, int lf, float scale,
+                        const bf16* mask, hipStream_t s) {
+  const int64_t n = (int64_t)d.nx[lf + 1] * d.ny[lf + 1] * (C / 8);
+  hipLaunchKernelGGL(k_down, dim3(nblk(n), (unsigned)nimg), dim3(256), 0, s, in, C, d.nx[lf], d.ny[lf], out,
+                     d.nx[lf + 1], d.ny[lf + 1], scale, mask);
+}
+static void up_launch(const Dims& d, int nimg, const bf16* in, bf16* out, int C, int lf, float scale, int accumulate,
+                      const bf16* mask, hipStream_t s) {
+  const int64_t n = (int64_t)d.nx[lf] * d.ny[lf] * (C / 8);
+  hipLaunchKernelGGL(k_up, dim3(nblk(n), (unsigned)nimg), dim3(256), 0, s, in, C, d.nx[lf + 1], d.ny[lf + 1], out,
+                     d.nx[lf], d.ny[lf], scale, accumulate, mask);
 }
 
 void unet_sync_bf16(UNet& net) {
@@ -725,34 +881,25 @@ void unet_forward(const UNet& net, UNetWork& ws, hipStream_t s, int nimg, int nx
   ensure_ws(ws, nimg, nx, ny);
   Dims d = dims_of(nimg, nx, ny);
   auto conv = [&](int l) {
-    const ConvSpec& c = kSpec[l];
-    const int lv = c.level;
-    const bf16* in = kIn[l] < 0 ? x : act(ws, kIn[l]);
-    conv_launch(in, c.ci, net.wb[l], net.b[l], act(ws, kOut[l]), c.co, nimg, d.nx[lv], d.ny[lv], 1, s);
+    const int lv = kSpec[l].level;
+    conv_launch(src_of(ws, kIn[l], x), net.wb[l], net.b[l], {act(ws, kOut[l]), nullptr, kSpec[l].co, 0}, nullptr, nimg,
+                d.nx[lv], d.ny[lv], 1, s);
   };
   auto down = [&](int a_in, int a_out, int lf) {
-    const int C = kActC[a_in];
-    hipLaunchKernelGGL(k_down, dim3(nblk(d.T[lf + 1] * C)), dim3(256), 0, s, act(ws, a_in), C, d.nx[lf], d.ny[lf],
-                       act(ws, a_out), d.nx[lf + 1], d.ny[lf + 1], nimg, 1.f);
+    down_launch(d, nimg, act(ws, a_in), act(ws, a_out), kActC[a_in], lf, 1.f, nullptr, s);
   };
   auto up = [&](int a_in, int a_out, int lc) {
-    const int C = kActC[a_in];
-    hipLaunchKernelGGL(k_up, dim3(nblk(d.T[lc - 1] * C)), dim3(256), 0, s, act(ws, a_in), C, d.nx[lc], d.ny[lc],
-                       act(ws, a_out), d.nx[lc - 1], d.ny[lc - 1], nimg, 1.f, 0);
-  };
-  auto cat = [&](int a, int b, int c, int lv) {
-    hipLaunchKernelGGL(k_concat, dim3(nblk(d.T[lv] * kActC[c])), dim3(256), 0, s, act(ws, a), kActC[a], act(ws, b),
-                       kActC[b], act(ws, c), d.T[lv]);
+    up_launch(d, nimg, act(ws, a_in), act(ws, a_out), kActC[a_in], lc - 1, 1.f, 0, nullptr, s);
   };
   conv(0); conv(1); down(A_S0, A_D1, 0);
   conv(2); conv(3); down(A_S1, A_D2, 1);
   conv(4); conv(5); down(A_S2, A_D3, 2);
   conv(6); conv(7);
-  up(A_B3, A_U2, 3); cat(A_U2, A_S2, A_C2, 2);
+  up(A_B3, A_U2, 3);
   conv(8); conv(9);
-  up(A_B4, A_U1, 2); cat(A_U1, A_S1, A_C1, 1);
+  up(A_B4, A_U1, 2);
   conv(10); conv(11);
-  up(A_B5, A_U0, 1); cat(A_U0, A_S0, A_C0, 0);
+  up(A_B5, A_U0, 1);
   conv(12); conv(13);
   hipLaunchKernelGGL(k_head_fwd, dim3(nblk(d.T[0])), dim3(256), 0, s, act(ws, A_B6), net.hw, net.hb, y, d.T[0]);
 }
@@ -800,7 +947,6 @@ static void ensure_scratch(UNetWork& ws, int64_t n) {
 
 void unet_backward(UNet& net, UNetWork& ws, hipStream_t s, int nimg, int nx, int ny, const bf16* x, const float* dy) {
   Dims d = dims_of(nimg, nx, ny);
-  bf16* dpre = (bf16*)ws.bufs[2 * A_NUM];
   // scratch: weight- and bias-gradient partials (WG_SCRATCH floats), or head
   // partials
   ensure_scratch(ws, WG_SCRATCH);
@@ -821,54 +967,44 @@ void unet_backward(UNet& net, UNetWork& ws, hipStream_t s, int nimg, int nx, int
       o += 9LL * kSpec[l].co * kSpec[l].ci + kSpec[l].co;
     }
   }
-  // conv layer backward: g(out) -> dpre -> dW, db, g(in)
+  // conv layer backward: the gradient before the ReLU (each pass that completes the
+  // gradient of a layer's output masks it) -> dW, db, g(in)
   auto conv_b = [&](int l, bool need_din) {
     const ConvSpec& c = kSpec[l];
     const int lv = c.level;
     const int64_t T = d.T[lv];
-    hipLaunchKernelGGL(k_relu_bwd, dim3(nblk(T * c.co)), dim3(256), 0, s, grd(ws, kOut[l]), act(ws, kOut[l]), dpre,
-                       T * c.co);
-    const bf16* in = kIn[l] < 0 ? x : act(ws, kIn[l]);
+    const bf16* dpre = grd(ws, kOut[l]);
+    const Src in = src_of(ws, kIn[l], x);
     int64_t per;
     const int64_t np = 9LL * c.co * c.ci + c.co;  // the layer's weights and bias
     const int64_t nb = pick_wgrad_blocks(T, np, &per);
     float* pw = ws.scratch;
     const dim3 g((unsigned)nb, (unsigned)(c.ci / 16));
     switch (c.co / 16) {
-      case 1: hipLaunchKernelGGL(k_conv_wgrad<1>, g, dim3(256), 0, s, dpre, in, c.ci, d.nx[lv], d.ny[lv], T, per, pw); break;
-      case 2: hipLaunchKernelGGL(k_conv_wgrad<2>, g, dim3(256), 0, s, dpre, in, c.ci, d.nx[lv], d.ny[lv], T, per, pw); break;
-      case 4: hipLaunchKernelGGL(k_conv_wgrad<4>, g, dim3(256), 0, s, dpre, in, c.ci, d.nx[lv], d.ny[lv], T, per, pw); break;
+      case 1: hipLaunchKernelGGL(k_conv_wgrad<1>, g, dim3(256), 0, s, dpre, in, d.nx[lv], d.ny[lv], T, per, pw); break;
+      case 2: hipLaunchKernelGGL(k_conv_wgrad<2>, g, dim3(256), 0, s, dpre, in, d.nx[lv], d.ny[lv], T, per, pw); break;
+      case 4: hipLaunchKernelGGL(k_conv_wgrad<4>, g, dim3(256), 0, s, dpre, in, d.nx[lv], d.ny[lv], T, per, pw); break;
       default: throw std::runtime_error("unsupported output channel count");
     }
     hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((np + 15) / 16)), dim3(256), 0, s, pw, (int)nb, np,
                        net.grad + off[l]);
     if (need_din)
-      conv_launch(dpre, c.co, net.wt[l], nullptr, grd(ws, kIn[l]), c.ci, nimg, d.nx[lv], d.ny[lv], 0, s);
-  };
-  auto split = [&](int ac, int au, int askip, int lv) {
-    hipLaunchKernelGGL(k_split, dim3(nblk(d.T[lv] * kActC[ac])), dim3(256), 0, s, grd(ws, ac), kActC[au],
-                       kActC[askip], grd(ws, au), grd(ws, askip), 0, d.T[lv]);
+      conv_launch({dpre, nullptr, c.co, 0}, net.wt[l], nullptr, grad_of(ws, kIn[l]),
+                  is_conv_out(kIn[l]) ? act(ws, kIn[l]) : nullptr, nimg, d.nx[lv], d.ny[lv], 0, s);
   };
   // g(b) = P^T g(u) = 4 R g(u)
   auto up_b = [&](int au, int ab, int lc) {
-    const int C = kActC[au];
-    hipLaunchKernelGGL(k_down, dim3(nblk(d.T[lc] * C)), dim3(256), 0, s, grd(ws, au), C, d.nx[lc - 1], d.ny[lc - 1],
-                       grd(ws, ab), d.nx[lc], d.ny[lc], nimg, 4.f);
+    down_launch(d, nimg, grd(ws, au), grd(ws, ab), kActC[au], lc - 1, 4.f, act(ws, ab), s);
   };
   // g(s) += R^T g(d) = P g(d) / 4
   auto down_b = [&](int ad, int as, int lf) {
-    const int C = kActC[ad];
-    hipLaunchKernelGGL(k_up, dim3(nblk(d.T[lf] * C)), dim3(256), 0, s, grd(ws, ad), C, d.nx[lf + 1], d.ny[lf + 1],
-                       grd(ws, as), d.nx[lf], d.ny[lf], nimg, 0.25f, 1);
+    up_launch(d, nimg, grd(ws, ad), grd(ws, as), kActC[ad], lf, 0.25f, 1, act(ws, as), s);
   };
   conv_b(13, true); conv_b(12, true);
-  split(A_C0, A_U0, A_S0, 0);
   up_b(A_U0, A_B5, 1);
   conv_b(11, true); conv_b(10, true);
-  split(A_C1, A_U1, A_S1, 1);
   up_b(A_U1, A_B4, 2);
   conv_b(9, true); conv_b(8, true);
-  split(A_C2, A_U2, A_S2, 2);
   up_b(A_U2, A_B3, 3);
   conv_b(7, true); conv_b(6, true);
   down_b(A_D3, A_S2, 2);
