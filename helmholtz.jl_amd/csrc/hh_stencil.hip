@@ -435,26 +435,35 @@ __global__ __launch_bounds__(256) void k_add_const(double* __restrict__ a, doubl
 }
 
 // ---- coarsest level: apply of the dense inverse (hh_dense.hip) ----
-// x_b = Ainv r_b in complex128 for every right-hand side.  One wavefront per
-// RT rows and DR right-hand sides: lanes stride the columns of the row-major
-// inverse (coalesced), each lane keeps RT x DR partial sums, wave shuffles
-// combine them (the same order of additions for every RT and DR).  The inverse
-// is re-read nrhs/DR times and r n/RT times.  UN column steps are loaded before
-// the first is used: with few right-hand sides a wavefront reads one or two rows
-// and nothing else hides the loads' latency.
+// x_b = Ainv r_b in complex128 for every right-hand side.  Bound by reading the
+// inverse from the Infinity Cache or HBM and r from L2.  A block takes RT rows and DR
+// right-hand sides; its 256 threads stride the columns of the row-major inverse
+// (coalesced), each keeps RT x DR partial sums, and wave shuffles and one exchange
+// through LDS combine them, in the same order of additions for every RT and DR.  The
+// four wavefronts split the columns, so a value of r serves RT rows from one load; with a
+// row to a wavefront r came from L2 DR times for each value of the inverse (2145 nodes
+// x 4 RHS: 22 us for 73 MB, now 15.6).  UN column steps are loaded before the first is used.
+// acc + a r in explicit fmas: every tile gives the same bits
+__device__ __forceinline__ cx<double> cmac(cx<double> acc, cx<double> a, cx<double> r) {
+  return mk<double>(fma(-a.im, r.im, fma(a.re, r.re, acc.re)), fma(a.im, r.re, fma(a.re, r.im, acc.im)));
+}
+
 template <typename T, int RT, int DR, int UN>
 __global__ __launch_bounds__(256) void k_dense_apply(const cx<double>* __restrict__ Arow, int n, int nrhs,
                                                      const cx<T>* __restrict__ r, cx<T>* __restrict__ x,
                                                      const int* __restrict__ skip) {
-  const int lane = threadIdx.x & 63;
-  const int i0 = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * RT;
+  constexpr int M = 2 * RT * DR;
+  __shared__ double sums[4][M];
+  const int lane = threadIdx.x & 63, wid = (int)(threadIdx.x >> 6);
+  const int i0 = (int)blockIdx.x * RT;
   const int rhs0 = blockIdx.y * DR;
-  if (i0 >= n) return;  // uniform per wavefront
   const int nr = min(DR, nrhs - rhs0);
-  const int ni = min(RT, n - i0);
-  bool live = !skip;
-  for (int k = 0; k < nr && !live; ++k) live = !skip[rhs0 + k];
-  if (!live) return;
+  if (skip) {
+    int done = 1;
+#pragma unroll
+    for (int k = 0; k < DR; ++k) done &= skip[rhs0 + min(k, nr - 1)] != 0;
+    if (done) return;
+  }
   const cx<double>* row[RT];
 #pragma unroll
   for (int a = 0; a < RT; ++a) row[a] = Arow + (int64_t)min(i0 + a, n - 1) * n;
@@ -466,43 +475,42 @@ __global__ __launch_bounds__(256) void k_dense_apply(const cx<double>* __restric
   for (int a = 0; a < RT; ++a)
 #pragma unroll
     for (int k = 0; k < DR; ++k) acc[a][k] = mk<double>(0.0, 0.0);
-  int j = lane;
-  for (; j + 64 * (UN - 1) < n; j += 64 * UN) {
-    cx<double> av[UN][RT], rv[UN][DR];
+  for (int j = threadIdx.x; j < n; j += 256 * UN) {
+    cx<double> av[UN][RT];
+    cx<T> rv[UN][DR];
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
+      const int ju = min(j + 256 * u, n - 1);  // a column past the last one: its values times 0
 #pragma unroll
-      for (int a = 0; a < RT; ++a) av[u][a] = row[a][j + 64 * u];
+      for (int a = 0; a < RT; ++a) av[u][a] = row[a][ju];
 #pragma unroll
-      for (int k = 0; k < DR; ++k) rv[u][k] = cvt<T, double>(rc[k][j + 64 * u]);
+      for (int k = 0; k < DR; ++k) rv[u][k] = rc[k][ju];
     }
 #pragma unroll
     for (int u = 0; u < UN; ++u)
 #pragma unroll
-      for (int a = 0; a < RT; ++a)
+      for (int k = 0; k < DR; ++k) {
+        const cx<double> rk = j + 256 * u < n ? cvt<T, double>(rv[u][k]) : mk<double>(0.0, 0.0);
 #pragma unroll
-        for (int k = 0; k < DR; ++k) acc[a][k] = acc[a][k] + av[u][a] * rv[u][k];
+        for (int a = 0; a < RT; ++a) acc[a][k] = cmac(acc[a][k], av[u][a], rk);
+      }
   }
-  for (; j < n; j += 64) {
-#pragma unroll
-    for (int a = 0; a < RT; ++a) {
-      const cx<double> av = row[a][j];
-#pragma unroll
-      for (int k = 0; k < DR; ++k) acc[a][k] = acc[a][k] + av * cvt<T, double>(rc[k][j]);
-    }
-  }
+  double v[M];
 #pragma unroll
   for (int a = 0; a < RT; ++a)
 #pragma unroll
     for (int k = 0; k < DR; ++k) {
-      double re = acc[a][k].re, im = acc[a][k].im;
-      for (int o = 32; o > 0; o >>= 1) {
-        re += __shfl_down(re, o, 64);
-        im += __shfl_down(im, o, 64);
-      }
-      if (lane == 0 && a < ni && k < nr && !(skip && skip[rhs0 + k]))
-        x[(int64_t)(rhs0 + k) * n + i0 + a] = cvt<double, T>(mk<double>(re, im));
+      v[2 * (a * DR + k)] = acc[a][k].re;
+      v[2 * (a * DR + k) + 1] = acc[a][k].im;
     }
+  WaveSums<M, 32>::run(v, lane, 0, M, [&](int q, double s) { sums[wid][q] = s; });
+  __syncthreads();
+  const int q = threadIdx.x;
+  if (q >= M) return;
+  const int a = (q >> 1) / DR, k = (q >> 1) % DR;
+  if (i0 + a >= n || k >= nr || (skip && skip[rhs0 + k])) return;
+  ((T*)x)[2 * ((int64_t)(rhs0 + k) * n + i0 + a) + (q & 1)] =
+      (T)(((sums[0][q] + sums[1][q]) + sums[2][q]) + sums[3][q]);
 }
 
 // ---- coarsest apply on MFMA (complex64 preconditioner) ----
@@ -765,30 +773,39 @@ void launch_add_const(double* a, double c, int64_t n, hipStream_t s) {
 template <typename T, int RT, int DR, int UN>
 static void dense_apply_go(const cx<double>* Ainv, int n, int nrhs, const cx<T>* r, cx<T>* x, const int* skip,
                            hipStream_t s) {
-  dim3 grid((unsigned)((n + 4 * RT - 1) / (4 * RT)), (unsigned)((nrhs + DR - 1) / DR));
+  dim3 grid((unsigned)((n + RT - 1) / RT), (unsigned)((nrhs + DR - 1) / DR));
   hipLaunchKernelGGL((k_dense_apply<T, RT, DR, UN>), grid, dim3(256), 0, s, Ainv, n, nrhs, r, x, skip);
 }
 
-// 4 rows x 4 RHS per wavefront read the inverse and r least often, but leave
-// 561 rows x 1 RHS with 36 blocks, three of whose four sums are padding: below
-// 1200 such wavefronts a wavefront takes one row and up to four RHS, and a single
-// RHS always has the one-row form.  Measured on MI355X, 4 x 4 form / this one,
-// with 14 us of copies and call around each: 561 nodes 1 RHS 26 / 18 us, 4 RHS
-// 28 / 20; 1183 nodes 8 RHS 36 / 28; 2145 nodes 1 RHS 44 / 29, 4 RHS 47 / 36,
-// 8 RHS 51 / 50; beyond the line 2145 nodes 12 RHS 56 / 62, 6305 nodes 2 RHS
-// 138 / 166.  6305 nodes 1 RHS: 134 / 134, the inverse at 5.3 TB/s.
+// Rows x right-hand sides per block.  Kernel times on MI355X in us, one-row (4 x 4)
+// wavefronts of before / now: 561 nodes 1 RHS 3.2 / 3.2, 4 RHS 5.1 / 4.5, 8 RHS 6.6 / 5.4;
+// 1183 nodes 1 RHS 5.6 / 4.4, 2 RHS 7.4 / 5.7, 4 RHS 10.0 / 6.7, 8 RHS 13.1 / 9.4;
+// 2145 nodes 1 RHS 14.6 / 13.1, 2 RHS 16.2 / 13.9, 4 RHS 21.9 / 15.6, 8 RHS 35.2 / 22.7.
+// More rows a block lose the small ones their blocks (561 nodes 4 RHS with 4 rows 5.3).
+// An inverse that the L2s hold is cheap to read again, r is not cheaper: tiles of 8 RHS
+// win beyond about 1600 nodes (1183 nodes x 8 RHS, 4 / 8 a tile: 9.4 / 11.1 us; 2145: 26.0 /
+// 22.7).  Past the Infinity Cache (n > 4096) the inverse comes from HBM, and four rows with
+// more columns in flight keep it busiest: 6305 nodes with the call 1 RHS 131 / 120 us,
+// 2 RHS 132 / 125, 4 RHS 147 / 140, 8 RHS 269 / 254.
 template <typename T>
 void launch_dense_apply(const cx<double>* Ainv, int64_t n, int nrhs, const cx<T>* r, cx<T>* x, const int* skip,
                         hipStream_t s) {
-  const int64_t waves = ((n + 3) / 4) * ((nrhs + 3) / 4);
-  if (nrhs == 1)
-    dense_apply_go<T, 1, 1, 8>(Ainv, (int)n, nrhs, r, x, skip, s);
-  else if (waves >= 1200)
-    dense_apply_go<T, 4, 4, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
-  else if (nrhs == 2)
-    dense_apply_go<T, 1, 2, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
-  else
-    dense_apply_go<T, 1, 4, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
+  if (n > 4096) {
+    if (nrhs == 1)
+      dense_apply_go<T, 2, 1, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
+    else if (nrhs == 2)
+      dense_apply_go<T, 4, 2, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
+    else
+      dense_apply_go<T, 4, 4, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
+  } else if (nrhs == 1) {
+    dense_apply_go<T, 2, 1, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
+  } else if (nrhs == 2) {
+    dense_apply_go<T, 2, 2, 2>(Ainv, (int)n, nrhs, r, x, skip, s);
+  } else if (nrhs <= 4 || n <= 1600) {
+    dense_apply_go<T, 2, 4, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
+  } else {
+    dense_apply_go<T, 2, 8, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
+  }
 }
 template void launch_dense_apply<double>(const cx<double>*, int64_t, int, const cx<double>*, cx<double>*,
                                          const int*, hipStream_t);
