@@ -1548,10 +1548,12 @@ void op_apply_device(hh_op* op, double shift, const void* xin, void* yout, int64
                                        nullptr, (cx<double>*)yout, op->d64, mm, sfac, nullptr, op->stream);
   } else if (prec == HH_C128)
     launch_stencil<double, double, double, M_APPLY>(op->g, (int)nrhs, (const cx<double>*)xin, nullptr,
-                                                    (cx<double>*)yout, op->d64, mm, sfac, 0.0, nullptr, op->stream);
+                                                    (cx<double>*)yout, op->d64, mm, sfac, 0.0, nullptr, op->stream, 0,
+                                                    nullptr, true);
   else
     launch_stencil<float, float, float, M_APPLY>(op->g, (int)nrhs, (const cx<float>*)xin, nullptr,
-                                                 (cx<float>*)yout, op->d32, mm, sfac, 0.0, nullptr, op->stream);
+                                                 (cx<float>*)yout, op->d32, mm, sfac, 0.0, nullptr, op->stream, 0, nullptr,
+                                                 true);
   HIPCK(hipGetLastError());
 }
 }  // namespace

@@ -8,12 +8,15 @@
 // terms (+ i s w^2 m_p for a shifted operator).
 //
 // Launch shape: 256 threads over consecutive positions of a row (2-D) or of
-// a plane (3-D), numbered across the grid so no lane idles at a ragged row
-// end; each thread marches a run of rows/planes along the slowest axis keeping
-// the previous/current/next values in registers, so x is read from HBM once;
-// in-plane neighbours come from the same or nearby cache lines.  The XCD-aware
+// a plane or a band of rows (3-D), numbered across the grid so no lane idles at a
+// ragged row end; each thread marches a run of rows/planes along the slowest axis
+// keeping the previous/current/next values in registers.  In-plane neighbours come
+// from the caches (small blocks) or from the neighbouring lanes.  The XCD-aware
 // block order groups right-hand sides that share the diagonal in L2.
 #include "hh_kernels.h"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace hh {
 
@@ -29,33 +32,22 @@ __device__ __forceinline__ cx<TD> node_diag(const cx<TD>* __restrict__ d, const 
   return dv;
 }
 
-// M_JACOBI: x + F (b - A x) with the level's precomputed damped-Jacobi factor
-// F = wj (d + diag of the Laplacian)^-1 when fj is given, else wj (b - A x) / Dtot
-template <typename TI, typename TO, typename TD, int MODE>
-__device__ __forceinline__ void finish(cx<TO>* __restrict__ yo, const cx<TO>* __restrict__ bo, int64_t p,
-                                       cx<TD> xc, cx<TD> Ax, cx<TD> Dtot, TD wj, const cx<TD>* __restrict__ fj) {
-  if (MODE == M_APPLY) {
-    yo[p] = cvt<TD, TO>(Ax);
-  } else if (MODE == M_RESID) {
-    cx<TD> bv = cvt<TO, TD>(bo[p]);
-    yo[p] = cvt<TD, TO>(bv - Ax);
-  } else {  // M_JACOBI
-    cx<TD> bv = cvt<TO, TD>(bo[p]);
-    cx<TD> r = bv - Ax;
-    if (fj) {
-      yo[p] = cvt<TD, TO>(xc + fj[p] * r);
-    } else {
-      cx<TD> up = r * cinv(Dtot);
-      yo[p] = cvt<TD, TO>(xc + wj * up);
-    }
-  }
+// What a mode makes of A x at one node; M_JACOBI: x + F (b - A x) with the level's
+// precomputed damped-Jacobi factor F = wj (d + diag of the Laplacian)^-1 when fj is
+// given, else wj (b - A x) / Dtot
+template <typename TO, typename TD, int MODE>
+__device__ __forceinline__ cx<TO> finish(cx<TD> xc, cx<TD> Ax, cx<TO> bo, cx<TD> Dtot, TD wj, bool has_f, cx<TD> f) {
+  if (MODE == M_APPLY) return cvt<TD, TO>(Ax);
+  const cx<TD> r = cvt<TO, TD>(bo) - Ax;
+  if (MODE == M_RESID) return cvt<TD, TO>(r);
+  return cvt<TD, TO>(xc + (has_f ? cmul_fma(f, r) : wj * cmul_fma(r, cinv(Dtot))));
 }
 
-// One thread per (column position, run of `rows` rows/planes): the positions
-// of a row (2-D) or of a plane (3-D) are numbered consecutively across the
-// whole grid, so a block of 256 threads covers 256 consecutive nodes with no
-// idle lanes at ragged row ends; each thread then marches its run along the
-// slowest axis keeping the previous/current/next values in registers.
+// Small blocks (x in L2): one thread per (column position, run of `rows`
+// rows/planes), the positions of a row (2-D) or of a plane (3-D) numbered
+// consecutively across the whole grid so no lane idles at a ragged row end; each
+// thread marches its run along the slowest axis keeping the previous/current/next
+// values in registers and reads its in-plane neighbours from the caches.
 template <typename TI, typename TO, typename TD, int MODE>
 __global__ __launch_bounds__(256) void k_stencil2d(Grid g, const cx<TI>* __restrict__ x,
                                                    const cx<TO>* __restrict__ b, cx<TO>* __restrict__ y,
@@ -73,7 +65,7 @@ __global__ __launch_bounds__(256) void k_stencil2d(Grid g, const cx<TI>* __restr
   const int j1 = min(j0 + rows, n2);
   const int64_t off = (int64_t)rhs * g.N;
   const cx<TI>* xr = x + off;
-  const cx<TO>* bo = b ? b + off : nullptr;
+  const cx<TO>* bo = MODE == M_APPLY ? nullptr : b + off;
   cx<TO>* yo = y + off;
   const int il = lo_nb(i, g.bc), ir = hi_nb(i, n1, g.bc);
   const TD ih1 = (TD)g.ih1, ih2 = (TD)g.ih2;
@@ -93,7 +85,8 @@ __global__ __launch_bounds__(256) void k_stencil2d(Grid g, const cx<TI>* __restr
     if (MODE == M_JACOBI && !fj) {
       Dtot.re += ldx + (TD)(g.ih2 * lap_diag1(j, n2, g.bc));
     }
-    finish<TI, TO, TD, MODE>(yo, bo, p, xc, Ax, Dtot, wj, fj);
+    yo[p] = finish<TO, TD, MODE>(xc, Ax, MODE == M_APPLY ? mk<TO>(0, 0) : bo[p], Dtot, wj, fj != nullptr,
+                                 MODE == M_JACOBI && fj ? fj[p] : mk<TD>(0, 0));
     xm = xc;
     xc = xp;
   }
@@ -117,7 +110,7 @@ __global__ __launch_bounds__(256) void k_stencil3d(Grid g, const cx<TI>* __restr
   const int64_t plane = (int64_t)n1 * n2;
   const int64_t off = (int64_t)rhs * g.N;
   const cx<TI>* xr = x + off;
-  const cx<TO>* bo = b ? b + off : nullptr;
+  const cx<TO>* bo = MODE == M_APPLY ? nullptr : b + off;
   cx<TO>* yo = y + off;
   const int il = lo_nb(i, g.bc), ir = hi_nb(i, n1, g.bc);
   const int jl = lo_nb(j, g.bc), jr = hi_nb(j, n2, g.bc);
@@ -143,9 +136,210 @@ __global__ __launch_bounds__(256) void k_stencil3d(Grid g, const cx<TI>* __restr
     if (MODE == M_JACOBI && !fj) {
       Dtot.re += ldxy + (TD)(g.ih3 * lap_diag1(k, n3, g.bc));
     }
-    finish<TI, TO, TD, MODE>(yo, bo, p, xc, Ax, Dtot, wj, fj);
+    yo[p] = finish<TO, TD, MODE>(xc, Ax, MODE == M_APPLY ? mk<TO>(0, 0) : bo[p], Dtot, wj, fj != nullptr,
+                                 MODE == M_JACOBI && fj ? fj[p] : mk<TD>(0, 0));
     xm = xc;
     xc = xp;
+  }
+}
+
+// neighbour lanes' values: lane l gets lane l - 1's (l + 1's), lane 0 (63) its own e
+__device__ __forceinline__ float lane_below(float v, float e) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(e), __float_as_int(v), 0x138, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_above(float v, float e) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(e), __float_as_int(v), 0x130, 0xf, 0xf, false));
+}
+__device__ __forceinline__ double lane_below(double v, double e) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(__double2hiint(e), __double2hiint(v), 0x138, 0xf, 0xf, false),
+                          __builtin_amdgcn_update_dpp(__double2loint(e), __double2loint(v), 0x138, 0xf, 0xf, false));
+}
+__device__ __forceinline__ double lane_above(double v, double e) {
+  return __hiloint2double(__builtin_amdgcn_update_dpp(__double2hiint(e), __double2hiint(v), 0x130, 0xf, 0xf, false),
+                          __builtin_amdgcn_update_dpp(__double2loint(e), __double2loint(v), 0x130, 0xf, 0xf, false));
+}
+
+// x neighbours of a thread's node from the wavefront's own values: lane l holds
+// position l of 64 consecutive ones, so the node to the left (right) is in lane
+// l - 1 (l + 1) unless the row ends there (mirror or self ghost) or the
+// wavefront does (lanes 0 and 63: one value read at `at`).
+struct XEdge {
+  int at;  // position in the row that lane 0 / 63 reads beside its own, -1: none
+  bool first, last, mirror;
+  __device__ __forceinline__ void init(int i, int n1, int bc) {
+    const int lane = threadIdx.x & 63;
+    first = i == 0;
+    last = i == n1 - 1;
+    mirror = bc == 2;
+    at = lane == 0 && !first ? i - 1 : (lane == 63 && !last ? i + 1 : -1);
+  }
+  template <typename T>
+  __device__ __forceinline__ void neighbours(cx<T> c, cx<T> e, cx<T>& l, cx<T>& r) const {
+    const cx<T> lo = mk<T>(lane_below(c.re, e.re), lane_below(c.im, e.im));
+    const cx<T> hi = mk<T>(lane_above(c.re, e.re), lane_above(c.im, e.im));
+    l = first ? (mirror ? hi : c) : lo;
+    r = last ? (mirror ? lo : c) : hi;
+  }
+};
+
+template <bool NT, typename T>
+__device__ __forceinline__ void put(cx<T>* q, cx<T> v) {
+  typedef T v2 __attribute__((ext_vector_type(2)));
+  const v2 u = {v.re, v.im};
+  if (NT)
+    __builtin_nontemporal_store(u, (v2*)q);
+  else
+    *(v2*)q = u;
+}
+
+// Larger blocks: bound by HBM and the Infinity Cache.  The gathering kernels above
+// read a plane's neighbours a step after the plane itself; by then part of it had
+// left L1 and L2, and x crossed L2's boundary 2.1 times (193 x 193 x 97 x 32 complex64:
+// 2.03 GB read for 0.93, 663 us).  Here every value that a thread needs is read once,
+// a step ahead, and kept: the x neighbours come from the neighbouring lanes' registers,
+// in 3-D a thread owns RY rows of a column and reads them and the row on either side.
+// NT: y is stored past the caches, which leaves their room to x.
+// 193 x 193 x 97 x 32 complex64: 663 -> 520 us a launch, 3.6 TB/s of x and y.
+// 2-D: one thread per (column position, run of `rows` rows) numbered as above.
+template <typename TI, typename TO, typename TD, int MODE, bool NT>
+__global__ __launch_bounds__(256) void k_march2d(Grid g, const cx<TI>* __restrict__ x,
+                                                   const cx<TO>* __restrict__ b, cx<TO>* __restrict__ y,
+                                                   const cx<TD>* __restrict__ d, const double* __restrict__ m,
+                                                   cx<double> sfac, TD wj, int rows, TileMap tm,
+                                                   const int* __restrict__ skip, const cx<TD>* __restrict__ fj) {
+  int bx, by, rhs;
+  tile_of(tm, bx, by, rhs);
+  if (skip && skip[rhs]) return;
+  const int n1 = g.n1, n2 = g.n2;
+  const unsigned item = (unsigned)bx * 256u + threadIdx.x, band = item / (unsigned)n1;
+  const int i = (int)(item - band * (unsigned)n1);
+  // lanes past the last band walk the last row and store nothing (their
+  // neighbours in the wavefront read their registers)
+  const bool own = (int64_t)band * rows < n2;
+  const int j0 = own ? (int)band * rows : n2 - 1;
+  const int64_t off = (int64_t)rhs * g.N;
+  const cx<TI>* xr = x + off;
+  const cx<TO>* bo = MODE == M_APPLY ? nullptr : b + off;
+  cx<TO>* yo = y + off;
+  XEdge ed;
+  ed.init(i, n1, g.bc);
+  const TD ih1 = (TD)g.ih1, ih2 = (TD)g.ih2;
+  const TD ldx = (TD)(g.ih1 * lap_diag1(i, n1, g.bc));
+  const cx<TI> zi = mk<TI>(0, 0);
+  cx<TI> xm = xr[(int64_t)lo_nb(j0, g.bc) * n1 + i];
+  cx<TI> xc = xr[(int64_t)j0 * n1 + i];
+  cx<TI> ec = ed.at >= 0 ? xr[(int64_t)j0 * n1 + ed.at] : zi;
+  for (int s = 0; s < rows; ++s) {
+    const int j = min(j0 + s, n2 - 1);
+    const int64_t row = (int64_t)j * n1, up = (int64_t)hi_nb(j, n2, g.bc) * n1;
+    const int64_t p = row + i;
+    const cx<TI> xp = xr[up + i];
+    const cx<TI> ep = ed.at >= 0 ? xr[up + ed.at] : zi;
+    const cx<TD> dv = node_diag<TD>(d, m, sfac, p);
+    const cx<TO> bv = MODE == M_APPLY ? mk<TO>(0, 0) : bo[p];
+    const cx<TD> fv = MODE == M_JACOBI && fj ? fj[p] : mk<TD>(0, 0);
+    cx<TI> xl, xrr;
+    ed.neighbours(xc, ec, xl, xrr);
+    const cx<TD> c = cvt<TI, TD>(xc);
+    const cx<TD> Ax = apply5(c, cvt<TI, TD>(xl), cvt<TI, TD>(xrr), cvt<TI, TD>(xm), cvt<TI, TD>(xp), ih1, ih2, dv);
+    cx<TD> Dtot = dv;
+    if (MODE == M_JACOBI && !fj) Dtot.re += ldx + (TD)(g.ih2 * lap_diag1(j, n2, g.bc));
+    if (own && j0 + s < n2) put<NT>(yo + p, finish<TO, TD, MODE>(c, Ax, bv, Dtot, wj, fj != nullptr, fv));
+    xm = xc;
+    xc = xp;
+    ec = ep;
+  }
+}
+
+// 3-D: a thread owns RY nodes of one in-plane column, rows j0 .. j0 + RY - 1, over a
+// run of `rows` planes; the columns of a band of RY rows are numbered consecutively
+// over the bands.
+template <typename TI, typename TO, typename TD, int MODE, int RY, bool NT>
+__global__ __launch_bounds__(256) void k_march3d(Grid g, const cx<TI>* __restrict__ x,
+                                                   const cx<TO>* __restrict__ b, cx<TO>* __restrict__ y,
+                                                   const cx<TD>* __restrict__ d, const double* __restrict__ m,
+                                                   cx<double> sfac, TD wj, int rows, TileMap tm,
+                                                   const int* __restrict__ skip, const cx<TD>* __restrict__ fj) {
+  int bx, by, rhs;
+  tile_of(tm, bx, by, rhs);
+  if (skip && skip[rhs]) return;
+  const int n1 = g.n1, n2 = g.n2, n3 = g.n3;
+  const unsigned item = (unsigned)bx * 256u + threadIdx.x, band = item / (unsigned)n1;
+  const int i = (int)(item - band * (unsigned)n1);
+  const int k0 = by * rows;
+  const int k1 = min(k0 + rows, n3);
+  // lanes past the last band walk the last row and store nothing
+  const int j0 = min((int)band * RY, n2 - 1);
+  const bool own = (int64_t)band * RY < n2;
+  const int64_t plane = (int64_t)n1 * n2;
+  const int64_t off = (int64_t)rhs * g.N;
+  const cx<TI>* xr = x + off;
+  const cx<TO>* bo = MODE == M_APPLY ? nullptr : b + off;
+  cx<TO>* yo = y + off;
+  XEdge ed;
+  ed.init(i, n1, g.bc);
+  const TD ih1 = (TD)g.ih1, ih2 = (TD)g.ih2, ih3 = (TD)g.ih3;
+  const TD ldx = (TD)(g.ih1 * lap_diag1(i, n1, g.bc));
+  // rows j0 - 1 .. j0 + RY with their ghosts (a row past the ghost row is never used)
+  int rw[RY + 2];
+#pragma unroll
+  for (int r = 0; r < RY + 2; ++r) {
+    const int t = j0 + r - 1;
+    rw[r] = (t < 0 ? lo_nb(0, g.bc) : (t < n2 ? t : (t == n2 ? hi_nb(n2 - 1, n2, g.bc) : n2 - 1))) * n1;
+  }
+  const cx<TI> zi = mk<TI>(0, 0);
+  cx<TI> xm[RY], xc[RY + 2], ec[RY];
+#pragma unroll
+  for (int r = 0; r < RY; ++r) {
+    xm[r] = xr[(int64_t)lo_nb(k0, g.bc) * plane + rw[r + 1] + i];
+    ec[r] = ed.at >= 0 ? xr[(int64_t)k0 * plane + rw[r + 1] + ed.at] : zi;
+  }
+#pragma unroll
+  for (int r = 0; r < RY + 2; ++r) xc[r] = xr[(int64_t)k0 * plane + rw[r] + i];
+  for (int k = k0; k < k1; ++k) {
+    const int64_t pl = (int64_t)k * plane;
+    const cx<TI>* xu = xr + (int64_t)hi_nb(k, n3, g.bc) * plane;
+    cx<TI> xp[RY + 2], ep[RY];
+    cx<TD> dv[RY], fv[RY];
+    cx<TO> bv[RY];
+#pragma unroll
+    for (int r = 0; r < RY; ++r) {
+      const int64_t p = pl + rw[r + 1] + i;
+      xp[r + 1] = xu[rw[r + 1] + i];
+      dv[r] = node_diag<TD>(d, m, sfac, p);
+      bv[r] = MODE == M_APPLY ? mk<TO>(0, 0) : bo[p];
+      fv[r] = MODE == M_JACOBI && fj ? fj[p] : mk<TD>(0, 0);
+    }
+    xp[0] = xp[RY + 1] = zi;
+#pragma unroll
+    for (int r = 0; r < RY; ++r) ep[r] = zi;
+    if (k + 1 < k1) {  // the next step's in-plane neighbours
+      xp[0] = xu[rw[0] + i];
+      xp[RY + 1] = xu[rw[RY + 1] + i];
+      if (ed.at >= 0)
+#pragma unroll
+        for (int r = 0; r < RY; ++r) ep[r] = xu[rw[r + 1] + ed.at];
+    }
+#pragma unroll
+    for (int r = 0; r < RY; ++r) {
+      cx<TI> xl, xrr;
+      ed.neighbours(xc[r + 1], ec[r], xl, xrr);
+      const cx<TD> c = cvt<TI, TD>(xc[r + 1]);
+      const cx<TD> Ax = apply7(c, cvt<TI, TD>(xl), cvt<TI, TD>(xrr), cvt<TI, TD>(xc[r]), cvt<TI, TD>(xc[r + 2]),
+                               cvt<TI, TD>(xm[r]), cvt<TI, TD>(xp[r + 1]), ih1, ih2, ih3, dv[r]);
+      cx<TD> Dtot = dv[r];
+      if (MODE == M_JACOBI && !fj)
+        Dtot.re += (TD)(ldx + (TD)(g.ih2 * lap_diag1(j0 + r, n2, g.bc))) + (TD)(g.ih3 * lap_diag1(k, n3, g.bc));
+      if (own && j0 + r < n2)
+        put<NT>(yo + pl + rw[r + 1] + i, finish<TO, TD, MODE>(c, Ax, bv[r], Dtot, wj, fj != nullptr, fv[r]));
+    }
+#pragma unroll
+    for (int r = 0; r < RY; ++r) {
+      xm[r] = xc[r + 1];
+      ec[r] = ep[r];
+    }
+#pragma unroll
+    for (int r = 0; r < RY + 2; ++r) xc[r] = xp[r];
   }
 }
 
@@ -611,71 +805,99 @@ void launch_dense_apply_mfma(const float* P, int64_t n, int nrhs, const cx<float
   hipLaunchKernelGGL(k_dense_apply_mfma, grid, dim3(256), 0, s, (const float4*)P, n2, ng, nrhs, (const float*)r,
                      (float*)x, skip);
 }
-// blocks: (positions of a row/plane x runs) / 256 along x, runs of planes along y (3-D)
-static inline TileMap stencil_map(const Grid& g, int nrhs, int rows) {
-  if (g.dim == 2) {
-    const int64_t items = (int64_t)g.n1 * ((g.n2 + rows - 1) / rows);
-    return make_tile_map((int)((items + 255) / 256), 1, nrhs);
-  }
-  const int64_t items = (int64_t)g.n1 * g.n2;
-  return make_tile_map((int)((items + 255) / 256), (g.n3 + rows - 1) / rows, nrhs);
+// Runs along the slowest axis for `cols` wavefronts per run: enough wavefronts to fill
+// 256 CUs, runs of about 16 (of nearly equal length) otherwise.
+static inline int pick_rows(int len, int64_t cols) {
+  int runs = std::max(1, (len + 8) / 16);
+  while (3 * runs <= len && cols * runs < 8192) runs *= 2;
+  return (len + runs - 1) / runs;
 }
 
-static inline int pick_rows(const Grid& g, int nrhs) {
-  // enough independent wavefronts to fill 256 CUs, long runs otherwise
-  const int64_t cols = ((int64_t)g.n1 * (g.dim == 3 ? g.n2 : 1) + 63) / 64 * nrhs;
-  const int len = g.dim == 3 ? g.n3 : g.n2;
-  int rows = 16;
-  while (rows > 2 && cols * ((len + rows - 1) / rows) < 8192) rows >>= 1;
-  return rows;
-}
-
+// x blocks up to 16 MB lie in the L2s, where re-reading the neighbours is cheaper than
+// the marches' longer start: 129 x 129 x 1 complex128 14.4 / 15.1 us a call (gathered /
+// marched), 61 x 50 x 33 x 8 complex64 18.4 / 19.7, 270 x 42 x 82 complex128 19.6 / 20.1.
+// Beyond: 513 x 257 x 8 complex128 20.7 / 19.7 us, 97 x 97 x 49 x 8 complex64 31.1 / 29.8,
+// 1025 x 513 x 64 complex64 167 / 133, 193 x 193 x 97 x 32 complex64 673 / 528,
+// x 12 complex128 504 / 380.  RY: complex128 2 / 4 rows 37 / 41 us (101 x 83 x 57 x 8),
+// complex64 566 / 528 us (193 x 193 x 97 x 32).  Stores past the caches (stream_out: y is
+// the caller's) help while x fits in about two Infinity Caches: 97 x 97 x 49 x 64
+// complex64 165 -> 115 us, 150 x 171 x 101 x 3 complex128 82 -> 71; with 925 MB of x
+// they cost 528 -> 551.
 template <typename TI, typename TO, typename TD, int MODE>
 void launch_stencil(const Grid& g, int nrhs, const cx<TI>* x, const cx<TO>* b, cx<TO>* y, const cx<TD>* d,
                     const double* m, cx<double> sfac, double wj, const int* skip, hipStream_t s, int rows_override,
-                    const cx<TD>* fj) {
-  const int rows = rows_override > 0 ? rows_override : pick_rows(g, nrhs);
-  const TileMap tm = stencil_map(g, nrhs, rows);
-  if (g.dim == 2)
-    hipLaunchKernelGGL((k_stencil2d<TI, TO, TD, MODE>), dim3(tm.T), dim3(256), 0, s, g, x, b, y, d, m, sfac,
-                       (TD)wj, rows, tm, skip, fj);
-  else
-    hipLaunchKernelGGL((k_stencil3d<TI, TO, TD, MODE>), dim3(tm.T), dim3(256), 0, s, g, x, b, y, d, m, sfac,
-                       (TD)wj, rows, tm, skip, fj);
+                    const cx<TD>* fj, bool stream_out) {
+  const bool d3 = g.dim == 3;
+  const int len = d3 ? g.n3 : g.n2;
+  const int64_t xbytes = (int64_t)sizeof(cx<TI>) * g.N * nrhs;
+  if (xbytes <= (16 << 20)) {
+    const int64_t cols = ((int64_t)g.n1 * (d3 ? g.n2 : 1) + 63) / 64 * nrhs;
+    int rows = 16;
+    while (rows > 2 && cols * ((len + rows - 1) / rows) < 8192) rows >>= 1;
+    if (rows_override > 0) rows = rows_override;
+    const int runs = (len + rows - 1) / rows;
+    const int64_t items = (int64_t)g.n1 * (d3 ? g.n2 : runs);
+    const TileMap tm = make_tile_map((int)((items + 255) / 256), d3 ? runs : 1, nrhs);
+    if (d3)
+      hipLaunchKernelGGL((k_stencil3d<TI, TO, TD, MODE>), dim3(tm.T), dim3(256), 0, s, g, x, b, y, d, m, sfac,
+                         (TD)wj, rows, tm, skip, fj);
+    else
+      hipLaunchKernelGGL((k_stencil2d<TI, TO, TD, MODE>), dim3(tm.T), dim3(256), 0, s, g, x, b, y, d, m, sfac,
+                         (TD)wj, rows, tm, skip, fj);
+    return;
+  }
+  constexpr int RY = sizeof(TI) == 4 ? 4 : 2;
+  const int64_t bands = d3 ? (g.n2 + RY - 1) / RY : 1;
+  const int rows = rows_override > 0 ? rows_override : pick_rows(len, ((int64_t)g.n1 * bands + 63) / 64 * nrhs);
+  const int runs = (len + rows - 1) / rows;
+  const int64_t items = (int64_t)g.n1 * (d3 ? bands : runs);
+  const TileMap tm = make_tile_map((int)((items + 255) / 256), d3 ? runs : 1, nrhs);
+  auto go = [&](auto nt) {
+    constexpr bool NT = decltype(nt)::value;
+    if (d3)
+      hipLaunchKernelGGL((k_march3d<TI, TO, TD, MODE, RY, NT>), dim3(tm.T), dim3(256), 0, s, g, x, b, y, d, m, sfac,
+                         (TD)wj, rows, tm, skip, fj);
+    else
+      hipLaunchKernelGGL((k_march2d<TI, TO, TD, MODE, NT>), dim3(tm.T), dim3(256), 0, s, g, x, b, y, d, m, sfac,
+                         (TD)wj, rows, tm, skip, fj);
+  };
+  if constexpr (MODE == M_APPLY)
+    if (stream_out && xbytes <= (512 << 20)) return go(std::true_type{});
+  go(std::false_type{});
 }
 
 template void launch_stencil<double, double, double, M_APPLY>(const Grid&, int, const cx<double>*,
                                                                const cx<double>*, cx<double>*,
                                                                const cx<double>*, const double*, cx<double>,
                                                                double, const int*, hipStream_t, int,
-                                                              const cx<double>*);
+                                                              const cx<double>*, bool);
 template void launch_stencil<double, double, double, M_RESID>(const Grid&, int, const cx<double>*,
                                                                const cx<double>*, cx<double>*,
                                                                const cx<double>*, const double*, cx<double>,
                                                                double, const int*, hipStream_t, int,
-                                                              const cx<double>*);
+                                                              const cx<double>*, bool);
 template void launch_stencil<double, double, double, M_JACOBI>(const Grid&, int, const cx<double>*,
                                                                 const cx<double>*, cx<double>*,
                                                                 const cx<double>*, const double*, cx<double>,
                                                                 double, const int*, hipStream_t, int,
-                                                              const cx<double>*);
+                                                              const cx<double>*, bool);
 template void launch_stencil<float, float, float, M_APPLY>(const Grid&, int, const cx<float>*, const cx<float>*,
                                                             cx<float>*, const cx<float>*, const double*,
                                                             cx<double>, double, const int*, hipStream_t, int,
-                                                              const cx<float>*);
+                                                              const cx<float>*, bool);
 template void launch_stencil<float, float, float, M_RESID>(const Grid&, int, const cx<float>*, const cx<float>*,
                                                             cx<float>*, const cx<float>*, const double*,
                                                             cx<double>, double, const int*, hipStream_t, int,
-                                                              const cx<float>*);
+                                                              const cx<float>*, bool);
 template void launch_stencil<float, float, float, M_JACOBI>(const Grid&, int, const cx<float>*, const cx<float>*,
                                                              cx<float>*, const cx<float>*, const double*,
                                                              cx<double>, double, const int*, hipStream_t, int,
-                                                              const cx<float>*);
+                                                              const cx<float>*, bool);
 template void launch_stencil<float, double, double, M_APPLY>(const Grid&, int, const cx<float>*,
                                                               const cx<double>*, cx<double>*,
                                                               const cx<double>*, const double*, cx<double>,
                                                               double, const int*, hipStream_t, int,
-                                                              const cx<double>*);
+                                                              const cx<double>*, bool);
 
 template <typename T>
 void launch_jacobi0(const Grid& g, int nrhs, const cx<T>* b, cx<T>* x, const cx<T>* f, const int* skip,
