@@ -273,7 +273,7 @@ __global__ __launch_bounds__(NT) void k_up_fused3(TileMap tm, int ytiles, int zr
   cx<T> xa0[KR], xa1[KR], xa2[KR], sa0[KR], sa1[KR], sa2[KR];
   cx<T> xn[KR], bn[KR], fn[KR];  // the next step's loads
   auto load_step = [&](int zz) {  // x of plane zz, b and F of plane zz - 1 (clamped: always in bounds)
-    const int64_t pz = (int64_t)min(zz, n3 - 1) * plane, pb = (int64_t)max(zz - 1, 0) * plane;
+    const int64_t pz = (int64_t)min(zz, n3 - 1) * plane, pb = (int64_t)max(min(zz, n3) - 1, 0) * plane;
 #pragma unroll
     for (int k = 0; k < KR; ++k) {
       xn[k] = xr[pz + m.po[k]];
