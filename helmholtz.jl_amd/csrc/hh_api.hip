@@ -677,20 +677,20 @@ struct Cycle {
   int ncorr_at(int l) const {
     return (S->p.cycle == 'W' && (S->p.wlevels <= 0 || l < S->p.wlevels)) ? 2 : 1;
   }
-  // fused 3-D up leg (last coarse correction + 2 post sweeps), complex64
+  // fused 3-D up leg (last coarse correction + 2 post sweeps)
   bool use_up3(const Level& L, int l) const {
-    return std::is_same<T, float>::value && S->p.fused && S->p.cycle != 'K' &&
-           S->p.relax_type == HH_RELAX_JAC && l + 1 < (int)S->lv.size() && post_at(l) == 2 && fused3_ok(L.g);
+    return S->p.fused && S->p.cycle != 'K' && S->p.relax_type == HH_RELAX_JAC && l + 1 < (int)S->lv.size() &&
+           post_at(l) == 2 && fused3_ok(L.g);
   }
-  // fused 3-D down leg (2 pre sweeps from zero + the residual), complex64
+  // fused 3-D down leg (2 pre sweeps from zero + the residual)
   bool use_down3(const Level& L, int l) const {
-    return std::is_same<T, float>::value && S->p.fused && S->p.cycle != 'K' &&
-           S->p.relax_type == HH_RELAX_JAC && l + 1 < (int)S->lv.size() && pre_at(l) == 2 && fused3_ok(L.g);
+    return S->p.fused && S->p.cycle != 'K' && S->p.relax_type == HH_RELAX_JAC && l + 1 < (int)S->lv.size() &&
+           pre_at(l) == 2 && fused3_ok(L.g);
   }
   // fused 3-D middle step of a W visit (prolongation + the next residual)
   bool use_mid3(const Level& L, int l) const {
-    return std::is_same<T, float>::value && S->p.fused && S->p.cycle != 'K' &&
-           S->p.relax_type == HH_RELAX_JAC && l + 1 < (int)S->lv.size() && fused3_ok(L.g);
+    return S->p.fused && S->p.cycle != 'K' && S->p.relax_type == HH_RELAX_JAC && l + 1 < (int)S->lv.size() &&
+           fused3_ok(L.g);
   }
   // damped-Jacobi sweeps before / after the coarse correction on level l
   int pre_at(int l) const { return S->p.per_level ? S->p.pre_l[l] : S->p.pre; }
@@ -845,14 +845,14 @@ struct Cycle {
     // in the coarse level's right-hand side
     const bool down3 = zero_init && use_down3(L, l);
     // kernel timing of the fused 3-D legs: algorithmic bytes as for the 2-D legs
-    const double s3 = sizeof(cx<float>), Nf3 = (double)L.g.N, act3 = S->kt_active;
+    const double s3 = sizeof(cx<T>), Nf3 = (double)L.g.N, act3 = S->kt_active;
     if (down3) {
       L.cur = first ? first : L.xa;
       Level& C = S->lv[l + 1];
       const bool td = S->kt.match(KT_DOWN, l);
       if (td) S->kt.begin(st);
-      launch_down_fused3(L.g, C.g, nrhs, (const cx<float>*)b, (const cx<float>*)L.d, (const cx<float>*)L.f,
-                         S->p.relax, (cx<float>*)L.cur, (cx<float>*)C.b, skip, st);
+      launch_down_fused3<T>(L.g, C.g, nrhs, b, (const cx<T>*)L.d, (const cx<T>*)L.f,
+                         S->p.relax, (cx<T>*)L.cur, (cx<T>*)C.b, skip, st);
       // b in, x2 and b_c out; d and F shared
       if (td) S->kt.end(st, act3 * (2 * Nf3 * s3 + (double)C.g.N * s3) + 2 * Nf3 * s3);
     } else if (zero_init) {
@@ -905,8 +905,8 @@ struct Cycle {
         void* o = other(L);
         const bool tm = S->kt.match(KT_MID, l);
         if (tm) S->kt.begin(st);
-        launch_mid_fused3(L.g, C.g, nrhs, (const cx<float>*)L.cur, (const cx<float>*)C.cur, (const cx<float>*)b,
-                          (const cx<float>*)L.d, (cx<float>*)o, (cx<float>*)C.b, skip, st);
+        launch_mid_fused3<T>(L.g, C.g, nrhs, (const cx<T>*)L.cur, (const cx<T>*)C.cur, b,
+                          (const cx<T>*)L.d, (cx<T>*)o, (cx<T>*)C.b, skip, st);
         // x and b in, x' out, the coarse correction in and b_c out; the diagonal shared
         if (tm) S->kt.end(st, act3 * (3 * Nf3 * s3 + 2 * (double)C.g.N * s3) + Nf3 * s3);
         L.cur = o;
@@ -919,8 +919,8 @@ struct Cycle {
       void* o = other(L);
       const bool tu = S->kt.match(KT_UP, l);
       if (tu) S->kt.begin(st);
-      launch_up_fused3(L.g, C.g, nrhs, (const cx<float>*)L.cur, (const cx<float>*)C.cur, (const cx<float>*)b,
-                       (const cx<float>*)L.f, S->p.relax, (cx<float>*)o, skip, st);
+      launch_up_fused3<T>(L.g, C.g, nrhs, (const cx<T>*)L.cur, (const cx<T>*)C.cur, b,
+                       (const cx<T>*)L.f, S->p.relax, (cx<T>*)o, skip, st);
       if (tu) S->kt.end(st, act3 * (3 * Nf3 * s3 + (double)C.g.N * s3) + Nf3 * s3);  // x, b in, x out; e_c; F
       L.cur = o;
       return;

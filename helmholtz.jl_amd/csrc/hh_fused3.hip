@@ -1,4 +1,4 @@
-// Fused multigrid legs for 3-D levels with mirror ghosts (BC = 2), complex64.
+// Fused multigrid legs for 3-D levels with mirror ghosts (BC = 2).
 //
 // Down leg (pre-smoothing from zero, then the restricted residual):
 //
@@ -38,6 +38,11 @@
 // and in-plane ghosts mirror (index -1 = 1, n = n - 2): a ghost node's value
 // is its mirror image's at every stage (up to the rounding of its neighbour
 // sums, taken in the other order), so every formula is the unfused one.
+//
+// Complex128 takes the same tile: 64 KB of LDS (down leg 96), 88-94 VGPRs, one block
+// per CU.  Against the separate kernels, which pass over the level 12 times a W
+// visit and take 10 launches, one W cycle on MI355X: 97 x 97 x 49 x 8 735 -> 497 us,
+// x 32 2082 -> 1358, 145 x 145 x 81 x 1 874 -> 729, 33 x 33 x 25 x 8 193 -> 159.
 #include "hh_kernels.h"
 
 namespace hh {
@@ -466,13 +471,17 @@ struct Runs3 {
   int ytiles, zrun;
   TileMap m;
 };
-Runs3 runs3(const Grid& g, int nrhs, int H) {
+// A complex128 block takes a CU for itself (LDS, 88-94 VGPRs), so more than 256 blocks
+// only recompute more planes: 97 x 97 x 49 x 8, one W cycle 497 us with at least
+// 256 blocks, 534 with 512, 560 with 1024 (145 x 113 x 65 x 3: 722 / 704 / 688).
+Runs3 runs3(const Grid& g, int nrhs, int H, bool c128) {
+  const int target = c128 ? 256 : 1024;
   Runs3 r;
   const int xtiles = (g.n1 + m3_tx(H) - 1) / m3_tx(H);
   r.ytiles = (g.n2 + m3_ty(H) - 1) / m3_ty(H);
   const int64_t per_run = (int64_t)xtiles * r.ytiles * nrhs;
   int runs = (g.n3 + 47) / 48;
-  int want = (int)std::min<int64_t>((1024 + per_run - 1) / per_run, std::max(1, g.n3 / 8));
+  int want = (int)std::min<int64_t>((target + per_run - 1) / per_run, std::max(1, g.n3 / 8));
   if (per_run * want < 256) want = (int)std::min<int64_t>((256 + per_run - 1) / per_run, (g.n3 + 3) / 4);
   runs = std::max(runs, want);
   r.zrun = (g.n3 + runs - 1) / runs;
@@ -482,28 +491,39 @@ Runs3 runs3(const Grid& g, int nrhs, int H) {
 }
 }  // namespace
 
-void launch_down_fused3(const Grid& gf, const Grid& gc, int nrhs, const cx<float>* b, const cx<float>* d,
-                         const cx<float>* f, double relax, cx<float>* xo, cx<float>* bco, const int* skip,
-                         hipStream_t s) {
-  const Runs3 r = runs3(gf, nrhs, 3);
-  hipLaunchKernelGGL((k_down_fused3<float, M3_NT>), dim3(r.m.T), dim3(M3_NT), 0, s, r.m, r.ytiles, r.zrun, gf, gc,
-                     b, d, f, xo, bco, skip, (float)(1.0 - relax));
+template <typename T>
+void launch_down_fused3(const Grid& gf, const Grid& gc, int nrhs, const cx<T>* b, const cx<T>* d, const cx<T>* f,
+                        double relax, cx<T>* xo, cx<T>* bco, const int* skip, hipStream_t s) {
+  const Runs3 r = runs3(gf, nrhs, 3, sizeof(T) == 8);
+  hipLaunchKernelGGL((k_down_fused3<T, M3_NT>), dim3(r.m.T), dim3(M3_NT), 0, s, r.m, r.ytiles, r.zrun, gf, gc, b, d, f,
+                     xo, bco, skip, (T)(1.0 - relax));
 }
 
-void launch_mid_fused3(const Grid& gf, const Grid& gc, int nrhs, const cx<float>* x, const cx<float>* ec,
-                       const cx<float>* b, const cx<float>* d, cx<float>* xo, cx<float>* bco, const int* skip,
-                       hipStream_t s) {
-  const Runs3 r = runs3(gf, nrhs, 2);
-  hipLaunchKernelGGL((k_mid_fused3<float, M3_NT>), dim3(r.m.T), dim3(M3_NT), 0, s, r.m, r.ytiles, r.zrun, gf, gc, x,
-                     ec, b, d, xo, bco, skip);
+template <typename T>
+void launch_mid_fused3(const Grid& gf, const Grid& gc, int nrhs, const cx<T>* x, const cx<T>* ec, const cx<T>* b,
+                       const cx<T>* d, cx<T>* xo, cx<T>* bco, const int* skip, hipStream_t s) {
+  const Runs3 r = runs3(gf, nrhs, 2, sizeof(T) == 8);
+  hipLaunchKernelGGL((k_mid_fused3<T, M3_NT>), dim3(r.m.T), dim3(M3_NT), 0, s, r.m, r.ytiles, r.zrun, gf, gc, x, ec, b,
+                     d, xo, bco, skip);
 }
 
-void launch_up_fused3(const Grid& gf, const Grid& gc, int nrhs, const cx<float>* x, const cx<float>* ec,
-                      const cx<float>* b, const cx<float>* f, double relax, cx<float>* xo, const int* skip,
-                      hipStream_t s) {
-  const Runs3 r = runs3(gf, nrhs, 2);
-  hipLaunchKernelGGL((k_up_fused3<float, M3_NT>), dim3(r.m.T), dim3(M3_NT), 0, s, r.m, r.ytiles, r.zrun, gf, gc, x,
-                     ec, b, f, xo, skip, (float)(1.0 - relax));
+template <typename T>
+void launch_up_fused3(const Grid& gf, const Grid& gc, int nrhs, const cx<T>* x, const cx<T>* ec, const cx<T>* b,
+                      const cx<T>* f, double relax, cx<T>* xo, const int* skip, hipStream_t s) {
+  const Runs3 r = runs3(gf, nrhs, 2, sizeof(T) == 8);
+  hipLaunchKernelGGL((k_up_fused3<T, M3_NT>), dim3(r.m.T), dim3(M3_NT), 0, s, r.m, r.ytiles, r.zrun, gf, gc, x, ec, b, f,
+                     xo, skip, (T)(1.0 - relax));
 }
+
+#define HH_FUSED3(T)                                                                                                  \
+  template void launch_down_fused3<T>(const Grid&, const Grid&, int, const cx<T>*, const cx<T>*, const cx<T>*,       \
+                                      double, cx<T>*, cx<T>*, const int*, hipStream_t);                              \
+  template void launch_mid_fused3<T>(const Grid&, const Grid&, int, const cx<T>*, const cx<T>*, const cx<T>*,        \
+                                     const cx<T>*, cx<T>*, cx<T>*, const int*, hipStream_t);                         \
+  template void launch_up_fused3<T>(const Grid&, const Grid&, int, const cx<T>*, const cx<T>*, const cx<T>*,         \
+                                    const cx<T>*, double, cx<T>*, const int*, hipStream_t);
+HH_FUSED3(float)
+HH_FUSED3(double)
+#undef HH_FUSED3
 
 }  // namespace hh
