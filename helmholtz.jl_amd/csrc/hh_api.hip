@@ -264,7 +264,8 @@ struct hh_solver {
   int* conv_d = nullptr;
   double* n2tmp = nullptr;
   double* res_d = nullptr;
-  int* h_done = nullptr;   // pinned host mirrors
+  int* h_done = nullptr;   // pinned host mirrors (h_done: two, taken in turn by the Arnoldi steps)
+  hipEvent_t ev_done[2] = {nullptr, nullptr};  // h_done's copies have arrived
   int* h_kact = nullptr;
   double* h_res = nullptr;
   double setup_time = 0, solve_time = 0;
@@ -371,6 +372,8 @@ struct hh_solver {
     nn_pix = npix;
   }
   ~hh_solver() {
+    for (hipEvent_t e : ev_done)
+      if (e) (void)hipEventDestroy(e);
     free_hier();
     free_learned();
     dfree(cap_buf);
@@ -593,7 +596,9 @@ void ensure_work(hh_solver* S, int nrhs) {
   S->conv_d = dalloc<int>(nrhs);
   S->n2tmp = dalloc<double>(nrhs);
   S->res_d = dalloc<double>(nrhs);
-  HIPCK(hipHostMalloc((void**)&S->h_done, sizeof(int) * nrhs, hipHostMallocDefault));
+  HIPCK(hipHostMalloc((void**)&S->h_done, 2 * sizeof(int) * nrhs, hipHostMallocDefault));
+  for (hipEvent_t& e : S->ev_done)
+    if (!e) HIPCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   HIPCK(hipHostMalloc((void**)&S->h_kact, sizeof(int) * nrhs, hipHostMallocDefault));
   HIPCK(hipHostMalloc((void**)&S->h_res, sizeof(double) * nrhs, hipHostMallocDefault));
   S->cap = nrhs;
@@ -1145,14 +1150,25 @@ void run_fgmres(hh_solver* S, int nrhs, hh_solve_stats* stats) {
       }
       HIPCK(hipGraphLaunch(S->gcycle, st));
     } else {
+      // The flags of step j are read while step j + 1 runs, so the queue never drains
+      // between two steps: reading each before the next was launched left the GPU idle
+      // 15-20 us a step (129 x 129, one RHS: 80 us a step).  The step that is launched
+      // past the last needed one finds every flag set and changes nothing.  Steps that
+      // the host itself looks at (captured training pairs, timed launches, the learned
+      // cycle) keep to their order.
+      const bool ahead = !S->cap_buf && !S->use_learned && S->kt.kernel == KT_NONE;
       for (int j = 0; j < K; ++j) {
         S->cap_now = S->cap_buf && nprec_cycle0 + j >= S->cap_lo && nprec_cycle0 + j < S->cap_hi && active == nrhs;
         S->kt_active = active;
         step(j);
-        HIPCK(hipMemcpyAsync(S->h_done, w.done, sizeof(int) * nrhs, hipMemcpyDeviceToHost, st));
-        HIPCK(hipStreamSynchronize(st));
+        HIPCK(hipMemcpyAsync(S->h_done + (j & 1) * S->cap, w.done, sizeof(int) * nrhs, hipMemcpyDeviceToHost, st));
+        HIPCK(hipEventRecord(S->ev_done[j & 1], st));
+        const int seen = ahead ? j - 1 : j;  // the step whose flags are read now
+        if (seen < 0) continue;
+        HIPCK(hipEventSynchronize(S->ev_done[seen & 1]));
+        const int* flags = S->h_done + (seen & 1) * S->cap;
         active = 0;
-        for (int b = 0; b < nrhs; ++b) active += S->h_done[b] == 0;
+        for (int b = 0; b < nrhs; ++b) active += flags[b] == 0;
         if (active == 0) break;
       }
       finish();
