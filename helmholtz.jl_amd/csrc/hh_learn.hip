@@ -15,6 +15,8 @@
 using namespace hh;
 
 namespace {
+constexpr int LOSS_PARTS = 256;  // blocks (and partial sums) of the loss: one per CU
+
 void ck2(hipError_t e, const char* w) {
   if (e != hipSuccess) throw std::runtime_error(std::string(w) + ": " + hipGetErrorString(e));
 }
@@ -129,7 +131,7 @@ void hh_unet::ensure_stage(int64_t npix) {
   y = dmal2<float>((size_t)npix * 2);
   dy = dmal2<float>((size_t)npix * 2);
   tgt = dmal2<float>((size_t)npix * 2);
-  loss_parts = dmal2<float>(256);
+  loss_parts = dmal2<float>(LOSS_PARTS);
   stage_pix = npix;
 }
 
@@ -223,10 +225,10 @@ int hh_unet_loss_grad(hh_unet* u, int nimg, int nx, int ny, const float* feats, 
     ck2(hipMemcpy(u->tgt, target, sizeof(float) * npix * 2, hipMemcpyHostToDevice), "upload");
     hipLaunchKernelGGL(k_feats_to_x16, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, u->stream, df, npix, u->x16);
     unet_forward(u->net, u->ws, u->stream, nimg, nx, ny, u->x16, u->y);
-    unet_mse(npix * 2, u->y, u->tgt, u->dy, u->loss_parts, 64, u->stream);
+    unet_mse(npix * 2, u->y, u->tgt, u->dy, u->loss_parts, LOSS_PARTS, u->stream);
     unet_backward(u->net, u->ws, u->stream, nimg, nx, ny, u->x16, u->dy);
     ck2(hipStreamSynchronize(u->stream), "backward");
-    float parts[64];
+    float parts[LOSS_PARTS];
     ck2(hipMemcpy(parts, u->loss_parts, sizeof(parts), hipMemcpyDeviceToHost), "loss");
     double s = 0;
     for (float v : parts) s += v;
@@ -291,7 +293,7 @@ int hh_unet_train(hh_unet* u, hh_dataset* d, int epochs, int batch, float lr, ui
     std::vector<int> order(d->n);
     std::iota(order.begin(), order.end(), 0);
     std::mt19937_64 rng(seed);
-    float parts[64];
+    float parts[LOSS_PARTS];
     for (int ep = 0; ep < epochs; ++ep) {
       std::shuffle(order.begin(), order.end(), rng);
       double acc = 0;
@@ -302,7 +304,7 @@ int hh_unet_train(hh_unet* u, hh_dataset* d, int epochs, int batch, float lr, ui
         hipLaunchKernelGGL(k_batch_prep, dim3((unsigned)((N * nb + 255) / 256)), dim3(256), 0, u->stream, d->r, d->e,
                            d->kh2, d->gw, d->h2, N, didx, dscale, nb, u->x16, u->tgt);
         unet_forward(u->net, u->ws, u->stream, nb, d->nx, d->ny, u->x16, u->y);
-        unet_mse(N * nb * 2, u->y, u->tgt, u->dy, u->loss_parts, 64, u->stream);
+        unet_mse(N * nb * 2, u->y, u->tgt, u->dy, u->loss_parts, LOSS_PARTS, u->stream);
         unet_backward(u->net, u->ws, u->stream, nb, d->nx, d->ny, u->x16, u->dy);
         unet_adam(u->net, lr, 0.9f, 0.999f, 1e-8f);
         ck2(hipMemcpyAsync(parts, u->loss_parts, sizeof(parts), hipMemcpyDeviceToHost, u->stream), "loss");

@@ -248,6 +248,7 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const bf16* __restrict__ dpr
   constexpr int COUT = 16 * NCO;
   constexpr int NTILE = 9 * NCO;
   constexpr int TPW = (NTILE + 3) / 4;
+  constexpr int BPX = WG_PX * COUT / 256;
   __shared__ __align__(16) bf16 sA[COUT * WG_LD];
   __shared__ __align__(16) bf16 sB[9 * 16 * WG_LD];
   __shared__ int sbase[WG_PX], si[WG_PX], sj[WG_PX];
@@ -309,9 +310,18 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const bf16* __restrict__ dpr
       store_px4(sB + (t * 16 + c8) * WG_LD + 4 * px4, v);
     }
     __syncthreads();
-    // bias gradient: one thread per output channel (ci block 0 only)
-    if (cib == 0 && threadIdx.x < COUT)
-      for (int px = 0; px < WG_PX; ++px) bsum += bf2f(sA[threadIdx.x * WG_LD + px]);
+    // bias gradient (ci block 0 only): a thread sums BPX pixels of a channel.  One thread
+    // per channel over all 64 held up the chunk's other wavefronts (27.2 us a launch of
+    // 16 channels x 266k pixels, 26.1 so).
+    if (cib == 0) {
+      const bf16* q = sA + (threadIdx.x % COUT) * WG_LD + (threadIdx.x / COUT) * BPX;
+#pragma unroll
+      for (int px = 0; px < BPX; px += 4) {
+        const s4 v = *(const s4*)(q + px);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bsum += bf2f((bf16)v[i]);
+      }
+    }
 #pragma unroll
     for (int k0 = 0; k0 < WG_PX; k0 += 16) {
 #pragma unroll
@@ -341,13 +351,25 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const bf16* __restrict__ dpr
         out[((int64_t)t * COUT + cob * 16 + kq + i) * cin + cib * 16 + m] = acc[ti][i];
     }
   }
-  if (cib == 0 && threadIdx.x < COUT) out[nw + threadIdx.x] = bsum;
+  if (cib == 0) {
+    float* sb = (float*)sA;  // the pixel groups' sums, added in order
+    __syncthreads();
+    sb[threadIdx.x] = bsum;
+    __syncthreads();
+    if (threadIdx.x < COUT) {
+      float b = 0.f;
+#pragma unroll
+      for (int h = 0; h < 256 / COUT; ++h) b += sb[h * COUT + threadIdx.x];
+      out[nw + threadIdx.x] = b;
+    }
+  }
 }
 
 // out[k] = sum_c part[c][k] in a fixed order: a block takes 16 outputs, its
 // 16 thread rows sum the partials c = row, row + 16, ... and the first row adds
-// the 16 row sums in order (one launch of n / 16 blocks instead of n / 256
-// threads each walking all partials: 3-5 us instead of ~20 us per layer)
+// the 16 row sums in order.  Bound by the latency of a thread's row of loads, so eight are
+// in flight at a time (833 partials of 2320 values: 17.1 us one by one, 5.7 so; the
+// training batch's fifteen launches 165 and 110 us).
 __global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ part, int nparts, int64_t n,
                                                    float* __restrict__ out) {
   __shared__ float sh[16][17];
@@ -355,7 +377,13 @@ __global__ __launch_bounds__(256) void k_sum_parts(const float* __restrict__ par
   const int64_t k = (int64_t)blockIdx.x * 16 + tx;
   float acc = 0.f;
   if (k < n)
-    for (int c = ty; c < nparts; c += 16) acc += part[(int64_t)c * n + k];
+    for (int c = ty; c < nparts; c += 128) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = c + 16 * u < nparts ? part[(int64_t)(c + 16 * u) * n + k] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc += v[u];
+    }
   sh[ty][tx] = acc;
   __syncthreads();
   if (ty == 0 && k < n) {
@@ -489,7 +517,9 @@ __global__ __launch_bounds__(256) void k_head_fwd(const bf16* __restrict__ x, co
   y[2 * p + 1] = y1;
 }
 
-// dx = hw^T dy (bf16) with x's own ReLU mask (x is a layer's output); per-block partial sums of dhw (2x16) and dhb (2)
+// dx = hw^T dy (bf16) with x's own ReLU mask (x is a layer's output); per-block partial sums of dhw (2x16) and dhb (2).
+// Bound by its one pass over x and dx: 16-byte accesses and a block per 512 pixels (266k
+// pixels: 64 blocks with 2-byte accesses 67 us, 505 blocks so 14.7).
 __global__ __launch_bounds__(256) void k_head_bwd(const bf16* __restrict__ x, const float* __restrict__ hw,
                                                   const float* __restrict__ dy, bf16* __restrict__ dx, int64_t npix,
                                                   int64_t chunk, float* __restrict__ part) {
@@ -500,14 +530,19 @@ __global__ __launch_bounds__(256) void k_head_bwd(const bf16* __restrict__ x, co
 #pragma unroll
   for (int k = 0; k < 34; ++k) acc[k] = 0.f;
   for (int64_t p = q0 + threadIdx.x; p < q1; p += 256) {
-    const float d0 = dy[2 * p], d1 = dy[2 * p + 1];
+    const float2 dp = ((const float2*)dy)[p];
+    const float d0 = dp.x, d1 = dp.y;
+    float v[16], g[16];
+    ld8(x + p * 16, *(float(*)[8])v);
+    ld8(x + p * 16 + 8, *(float(*)[8])(v + 8));
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
-      const float v = bf2f(x[p * 16 + c]);
-      acc[c] += d0 * v;
-      acc[16 + c] += d1 * v;
-      dx[p * 16 + c] = v > 0.f ? f2bf(hw[c] * d0 + hw[16 + c] * d1) : (bf16)0;
+      acc[c] += d0 * v[c];
+      acc[16 + c] += d1 * v[c];
+      g[c] = v[c] > 0.f ? hw[c] * d0 + hw[16 + c] * d1 : 0.f;
     }
+    st8(dx + p * 16, *(const float(*)[8])g, nullptr);
+    st8(dx + p * 16 + 8, *(const float(*)[8])(g + 8), nullptr);
     acc[32] += d0;
     acc[33] += d1;
   }
@@ -905,9 +940,9 @@ void unet_forward(const UNet& net, UNetWork& ws, hipStream_t s, int nimg, int nx
 }
 
 static int64_t pick_chunks(int64_t total, int64_t* chunk) {
-  int64_t nch = total / 4096;
+  int64_t nch = total / 512;
   if (nch < 1) nch = 1;
-  if (nch > 64) nch = 64;
+  if (nch > 512) nch = 512;
   int64_t c = (total + nch - 1) / nch;
   c = (c + 15) / 16 * 16;
   *chunk = c;
