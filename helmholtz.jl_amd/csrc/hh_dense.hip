@@ -21,6 +21,16 @@
 // updates as well.  Set-up time of a solver on MI355X (hierarchy included),
 // rank-1 form / this one: 561 nodes 7.0 / 2.0 ms, 1183 nodes 23.5 / 7.0 ms,
 // 2145 nodes 62 / 17 ms, 8385 nodes 2943 / 371 ms.
+//
+// The operator is banded in its node order (offsets up to bw = n1, in 3-D n1 n2), and
+// rows not yet used keep at most bw columns to their left and 2 bw to their right.  Up to
+// bw = 224 the elimination uses that (gj_band): a block's pivots lie in a window of
+// 32 + bw rows that one workgroup eliminates at once (k_gj_window: 32 columns in
+// 44-58 us instead of eight panels and updates in 160; bound by its barriers and LDS
+// reads, 1.4-1.8 us a column), the rows used before take one small product (k_gj_rows),
+// and the rank-32 update stops at column ke + 2 bw.  Panel form / this one: 1183 nodes
+// (13 x 13 x 7) 6.7 / 4.5 ms, 2145 nodes 16.8 / 8.1 ms, 3201 nodes 32 / 15 ms, 8385
+// nodes 371 / 116 ms; 561 nodes 1.9 / 1.8 ms.
 #include <algorithm>
 
 #include "hh_kernels.h"
@@ -206,11 +216,108 @@ __global__ __launch_bounds__(1024) void k_gj_panel(cx<double>* __restrict__ M, i
   }
 }
 
+// Block of columns kb .. kb + w - 1 (w <= 32) of a banded matrix: with node offsets of at
+// most bw, the rows not yet used that reach into the block lie in the window kb .. kb +
+// wr - 1, wr = 32 + bw at most, so the pivots are found and eliminated there: one
+// workgroup, four threads a row with eight columns each in registers.  The window's
+// rows get the panel's values, rows kb .. kb + w - 1 among them M_KK^-1; the rows used
+// before follow in k_gj_rows, all others are zero.  Same pivots as k_gj_panel's.
+__global__ __launch_bounds__(1024) void k_gj_window(cx<double>* __restrict__ M, int n, int kb, int w, int wr,
+                                                    GjPerm* __restrict__ pout) {
+  __shared__ unsigned long long key[GJ_NB];
+  __shared__ cx<double> rowp[GJ_NB], rowk[GJ_NB], pinv;
+  __shared__ int pvs[GJ_NB];
+  const int t = threadIdx.x, lane = t & 63, row = t >> 2, grp = t & 3;
+  const bool in = row < wr;
+  if (t < GJ_NB) key[t] = 0ull;
+  cx<double> a[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int c = grp * 8 + q;
+    a[q] = in && c < w ? M[(int64_t)(kb + c) * n + kb + row] : mk<double>(0.0, 0.0);
+  }
+  __syncthreads();
+  for (int g = 0; g < 4; ++g) {
+#pragma unroll
+    for (int q0 = 0; q0 < 8; ++q0) {
+      const int c = 8 * g + q0;
+      if (c >= w) break;
+      unsigned long long best = 0ull;
+      if (grp == g && row >= c && in)
+        best = ((unsigned long long)__double_as_longlong(cabs2(a[q0])) & ~16383ull) | (unsigned)(16383 - (kb + row));
+      best = wave_max(best);
+      if (lane == 63) atomicMax(&key[c], best);
+      // this row's value in column c, held by the group's thread g
+      const int from = (lane & ~3) | g;
+      const cx<double> own = mk<double>(__shfl(a[q0].re, from, 64), __shfl(a[q0].im, from, 64));
+      const cx<double> rec = cinv(a[q0]);  // ready, off the chain, should this be the pivot
+      __syncthreads();
+      const int p = 16383 - (int)(key[c] & 16383ull) - kb;
+      if (row == p)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) rowp[grp * 8 + q] = a[q];
+      if (row == p && grp == g) pinv = rec;
+      if (row == c)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) rowk[grp * 8 + q] = a[q];
+      if (t == 0) pvs[c] = kb + p;
+      __syncthreads();
+      const cx<double> inv = pinv;
+      cx<double> f = own;
+      if (row == p) {  // (one wavefront's branch: the others leave LDS alone)
+        f = rowk[c];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) a[q] = rowk[grp * 8 + q];
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const cx<double> pq = rowp[grp * 8 + q] * inv;
+        a[q] = row == c ? pq : a[q] - f * pq;
+      }
+      if (grp == g) a[q0] = row == c ? inv : mk<double>(0.0, 0.0) - f * inv;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int c = grp * 8 + q;
+    if (in && c < w) M[(int64_t)(kb + c) * n + kb + row] = a[q];
+  }
+  if (t < 64) gj_net(kb, w, lane < w ? pvs[lane] : 0, pout);
+}
+
+// Rows used before the block: M_IK' = -M_IK M_KK^-1, a block of 256 threads 64 rows,
+// eight columns a thread, M_KK^-1 (rows kb .. of the panel) in LDS.
+__global__ __launch_bounds__(256) void k_gj_rows(cx<double>* __restrict__ M, int n, int kb, int w) {
+  __shared__ cx<double> B[GJ_NB][GJ_NB];
+  const int t = threadIdx.x, grp = t >> 6;
+  for (int e = t; e < GJ_NB * GJ_NB; e += 256) {
+    const int l = e % GJ_NB, c = e / GJ_NB;
+    B[l][c] = l < w && c < w ? M[(int64_t)(kb + c) * n + kb + l] : mk<double>(0.0, 0.0);
+  }
+  const int i = blockIdx.x * 64 + (t & 63), r = min(i, kb - 1);
+  __syncthreads();
+  cx<double> acc[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) acc[q] = mk<double>(0.0, 0.0);
+#pragma unroll 8
+  for (int l = 0; l < GJ_NB; ++l) {
+    const cx<double> v = M[(int64_t)(kb + min(l, w - 1)) * n + r];  // (past the last: times a zero row)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) acc[q] = acc[q] - v * B[l][grp * 8 + q];
+  }
+  __syncthreads();  // every thread of a row has read it
+  if (i >= kb) return;
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (grp * 8 + q < w) M[(int64_t)(kb + grp * 8 + q) * n + i] = acc[q];
+}
+
 // Columns J of [s0, s1) outside the eliminated columns [k0, k0 + kw), CB whole
-// columns per block: the exchange, then M_J = (M_J, rows K zero) + panel M_KJ.
+// columns per block: the exchange, then M_J = (M_J, rows K zero) + panel M_KJ in the
+// first nr rows (the panel is zero below).
 template <int KM, int CB, int NT>
-__global__ __launch_bounds__(NT) void k_gj_update(cx<double>* __restrict__ M, int n, int k0, int kw, int s0, int s1,
-                                                   const GjPerm* __restrict__ pp) {
+__global__ __launch_bounds__(NT) void k_gj_update(cx<double>* __restrict__ M, int n, int nr, int k0, int kw, int s0,
+                                                   int s1, const GjPerm* __restrict__ pp) {
   __shared__ cx<double> Rk[KM][CB];
   __shared__ cx<double> V[2 * KM][CB];
   const int t = threadIdx.x;
@@ -241,8 +348,8 @@ __global__ __launch_bounds__(NT) void k_gj_update(cx<double>* __restrict__ M, in
   }
   const cx<double>* __restrict__ P = M + (int64_t)k0 * n;
   // two rows at a time: an M_KJ value read from LDS serves both
-  for (int r0 = t; r0 < n; r0 += 2 * NT) {
-    const int r[2] = {r0, min(r0 + NT, n - 1)};
+  for (int r0 = t; r0 < nr; r0 += 2 * NT) {
+    const int r[2] = {r0, min(r0 + NT, nr - 1)};
     cx<double> acc[2][CB];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -265,7 +372,7 @@ __global__ __launch_bounds__(NT) void k_gj_update(cx<double>* __restrict__ M, in
     for (int c = 0; c < CB; ++c)
       if (q0 + c < total) {
         col[c][r[0]] = acc[0][c];
-        if (r0 + NT < n) col[c][r[1]] = acc[1][c];
+        if (r0 + NT < nr) col[c][r[1]] = acc[1][c];
       }
   }
 }
@@ -333,15 +440,32 @@ void gj_run(cx<double>* M, int n, const GjWork& wk, hipStream_t s) {
                          blocked ? wk.inner : blk, blocked && k0 + w == ke ? blk : nullptr);
       if (!blocked) {
         if (n > w)
-          hipLaunchKernelGGL((k_gj_update<W, 2, 256>), dim3((n - w + 1) / 2), dim3(256), 0, s, M, n, k0, w, 0, n, blk);
+          hipLaunchKernelGGL((k_gj_update<W, 2, 256>), dim3((n - w + 1) / 2), dim3(256), 0, s, M, n, n, k0, w, 0, n, blk);
       } else if (ke - kb > w) {  // the block's other columns
-        hipLaunchKernelGGL((k_gj_update<W, 1, 1024>), dim3(ke - kb - w), dim3(1024), 0, s, M, n, k0, w, kb, ke,
+        hipLaunchKernelGGL((k_gj_update<W, 1, 1024>), dim3(ke - kb - w), dim3(1024), 0, s, M, n, n, k0, w, kb, ke,
                            wk.inner);
       }
     }
     if (blocked && n > ke - kb)
-      hipLaunchKernelGGL((k_gj_update<GJ_NB, 4, 256>), dim3((n - (ke - kb) + 3) / 4), dim3(256), 0, s, M, n, kb,
+      hipLaunchKernelGGL((k_gj_update<GJ_NB, 4, 256>), dim3((n - (ke - kb) + 3) / 4), dim3(256), 0, s, M, n, n, kb,
                          ke - kb, 0, n, blk);
+  }
+  hipLaunchKernelGGL(k_gj_order, dim3(1), dim3(64), sizeof(int) * n, s, n, nlist, wk.blocks, wk.pi);
+}
+
+// The banded elimination: per 32 columns one window, the rows used before and a rank-32
+// update of the columns that the rows in use reach (ke + 2 bw).
+constexpr int GJ_WINDOW = 256;  // rows of a window: 1024 threads
+void gj_band(cx<double>* M, int n, int bw, const GjWork& wk, hipStream_t s) {
+  int nlist = 0;
+  for (int kb = 0; kb < n; kb += GJ_NB, ++nlist) {
+    const int w = std::min(GJ_NB, n - kb), wr = std::min(n - kb, GJ_NB + bw);
+    const int nr = kb + wr, s1 = std::min(n, kb + w + 2 * bw);
+    hipLaunchKernelGGL(k_gj_window, dim3(1), dim3((4 * wr + 63) / 64 * 64), 0, s, M, n, kb, w, wr, wk.blocks + nlist);
+    if (kb > 0) hipLaunchKernelGGL(k_gj_rows, dim3((kb + 63) / 64), dim3(256), 0, s, M, n, kb, w);
+    if (s1 > w)
+      hipLaunchKernelGGL((k_gj_update<GJ_NB, 4, 256>), dim3((s1 - w + 3) / 4), dim3(256), 0, s, M, n, nr, kb, w, 0, s1,
+                         wk.blocks + nlist);
   }
   hipLaunchKernelGGL(k_gj_order, dim3(1), dim3(64), sizeof(int) * n, s, n, nlist, wk.blocks, wk.pi);
 }
@@ -365,8 +489,11 @@ void launch_dense_inverse(const Grid& g, const cx<double>* d, cx<double>* M2, vo
   wk.blocks = wk.inner + 1;
   launch_zero<double>(M, (int64_t)n * n, s);
   hipLaunchKernelGGL(k_dense_assemble, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g, d, M);
+  const int64_t bw = (int64_t)g.n1 * (g.dim == 3 ? g.n2 : 1);  // largest node offset of a row
   // columns per panel so that a thread's rows fit its 128 registers
-  if (n <= 1024)
+  if (bw + GJ_NB <= GJ_WINDOW)
+    gj_band(M, n, (int)bw, wk, s);
+  else if (n <= 1024)
     gj_run<8, 1>(M, n, wk, s);
   else if (n <= 2048)
     gj_run<6, 2>(M, n, wk, s);
