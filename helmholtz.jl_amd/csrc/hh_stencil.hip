@@ -715,7 +715,7 @@ __global__ __launch_bounds__(256) void k_dense_apply(const cx<double>* __restric
 // group g, step u (0..3) of v_mfma_f32_16x16x4_f32 gives lane l the column
 // k = 16g + 4(l/16) + u (a permutation of the group, the same for A and r), so
 // a lane reads its four A entries as one packed float4 and its four r entries
-// as two aligned float2.  A_R is packed once, in fp32: block (R, g), lane l
+// as another.  A_R is packed once, in fp32: block (R, g), lane l
 // holds row 16R + l % 16, columns 16g + 4(l/16) + 0..3 (zero beyond 2n).
 __global__ __launch_bounds__(256) void k_pack_inv_mfma(const cx<double>* __restrict__ Arow, int n, int ng, int nrb,
                                                        float4* __restrict__ P) {
@@ -742,7 +742,11 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // one block per 16 x 16 tile of the real-ified result (16 real rows, 16 RHS);
 // its four wavefronts take every fourth K-group and their partial tiles are
-// summed through LDS in a fixed order (deterministic)
+// summed through LDS in a fixed order (deterministic).  Bound by the address unit: a B
+// operand is 16 columns apart for 16 lanes, so it is one 16-byte load of four k and not
+// two of 8 (561 nodes x 256 RHS 34.8 -> 17.0 us, 1183 x 32 28.4 -> 20.4, 2145 x 256
+// 391 -> 195, 97 TFLOP/s; gfx950 takes 16-byte loads at 8-byte alignment).
+template <int UN>
 __global__ __launch_bounds__(256) void k_dense_apply_mfma(const float4* __restrict__ P, int n2, int ng, int nrhs,
                                                           const float* __restrict__ r, float* __restrict__ x,
                                                           const int* __restrict__ skip) {
@@ -760,18 +764,41 @@ __global__ __launch_bounds__(256) void k_dense_apply_mfma(const float4* __restri
   const int kl = lane >> 4;
   const float4* __restrict__ Pb = P + (int64_t)R * ng * 64 + lane;
   // n2 is even, so every column starts 8-byte aligned
-  const float2* __restrict__ rc = (const float2*)(r + (int64_t)(colok ? col : 0) * n2);
+  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(8)));
+  const float* __restrict__ rc = r + (int64_t)(colok ? col : 0) * n2;
   f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-  for (int g = wv; g < ng; g += 4) {
+  int g = wv;
+  if constexpr (UN > 1)  // whole groups, UN of them in flight; then what is left one by one
+    for (const int whole = n2 / 16; g + 4 * (UN - 1) < whole; g += 4 * UN) {
+      float4 av[UN];
+      f32x4u b[UN];
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+        av[u] = Pb[(int64_t)(g + 4 * u) * 64];
+        b[u] = *(const f32x4u*)(rc + (g + 4 * u) * 16 + 4 * kl);
+      }
+#pragma unroll
+      for (int u = 0; u < UN; ++u) {
+        acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u].x, b[u].x, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u].y, b[u].y, acc1, 0, 0, 0);
+        acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u].z, b[u].z, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u].w, b[u].w, acc1, 0, 0, 0);
+      }
+    }
+  for (; g < ng; g += 4) {
     const float4 av = Pb[(int64_t)g * 64];
     const int k = g * 16 + 4 * kl;
-    const float2 z2 = make_float2(0.f, 0.f);
-    const float2 b01 = (colok && k < n2) ? rc[k >> 1] : z2;
-    const float2 b23 = (colok && k + 2 < n2) ? rc[(k >> 1) + 1] : z2;
-    acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.x, b01.x, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.y, b01.y, acc1, 0, 0, 0);
-    acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.z, b23.x, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.w, b23.y, acc1, 0, 0, 0);
+    f32x4u b = {0.f, 0.f, 0.f, 0.f};
+    if (colok && k + 4 <= n2) {
+      b = *(const f32x4u*)(rc + k);
+    } else if (colok && k < n2) {  // the last group of 2n = 2 mod 4
+      b.x = rc[k];
+      b.y = rc[k + 1];
+    }
+    acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.x, b.x, acc0, 0, 0, 0);
+    acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.y, b.y, acc1, 0, 0, 0);
+    acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.z, b.z, acc0, 0, 0, 0);
+    acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(av.w, b.w, acc1, 0, 0, 0);
   }
   const f32x4 acc = acc0 + acc1;
   if (wv > 0) part[wv - 1][lane] = acc;
@@ -802,8 +829,15 @@ void launch_dense_apply_mfma(const float* P, int64_t n, int nrhs, const cx<float
                              hipStream_t s) {
   const int n2 = (int)(2 * n), ng = (n2 + 15) / 16, nrb = (n2 + 15) / 16;
   dim3 grid((unsigned)nrb, (unsigned)((nrhs + 15) / 16));
-  hipLaunchKernelGGL(k_dense_apply_mfma, grid, dim3(256), 0, s, (const float4*)P, n2, ng, nrhs, (const float*)r,
-                     (float*)x, skip);
+  // two K-groups in flight where the blocks are too few to hide a load's latency (one / two,
+  // us: 561 nodes x 48 RHS, 213 blocks 10.4 / 7.0; 1183 x 64, 592 blocks 22.8 / 20.1; 2145 x
+  // 48, 807 blocks 46.5 / 46.8; 561 x 256, 1136 blocks 16.4 / 17.5)
+  if ((int64_t)grid.x * grid.y < 800)
+    hipLaunchKernelGGL(k_dense_apply_mfma<2>, grid, dim3(256), 0, s, (const float4*)P, n2, ng, nrhs, (const float*)r,
+                       (float*)x, skip);
+  else
+    hipLaunchKernelGGL(k_dense_apply_mfma<1>, grid, dim3(256), 0, s, (const float4*)P, n2, ng, nrhs, (const float*)r,
+                       (float*)x, skip);
 }
 // Runs along the slowest axis for `cols` wavefronts per run: enough wavefronts to fill
 // 256 CUs, runs of about 16 (of nearly equal length) otherwise.
