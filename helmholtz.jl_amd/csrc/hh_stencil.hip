@@ -192,14 +192,16 @@ __device__ __forceinline__ void put(cx<T>* q, cx<T> v) {
     *(v2*)q = u;
 }
 
-// Larger blocks: bound by HBM and the Infinity Cache.  The gathering kernels above
-// read a plane's neighbours a step after the plane itself; by then part of it had
-// left L1 and L2, and x crossed L2's boundary 2.1 times (193 x 193 x 97 x 32 complex64:
-// 2.03 GB read for 0.93, 663 us).  Here every value that a thread needs is read once,
-// a step ahead, and kept: the x neighbours come from the neighbouring lanes' registers,
-// in 3-D a thread owns RY rows of a column and reads them and the row on either side.
+// Larger blocks: the gathering kernels above load five (2-D: three) values of x a node
+// and read a plane's neighbours a step after the plane itself, when part of it has left
+// L1 and L2: 193 x 193 x 97 x 32 complex64 took 55.7 million L2 requests and read 2.03 GB
+// for 0.93 (663 us).  Here every value that a thread needs is loaded once, a step ahead,
+// and kept: the x neighbours come from the neighbouring lanes' registers, in 3-D a thread
+// owns RY rows of a column and reads them and the row on either side.  39.1 million
+// requests, 520 us, 3.6 TB/s of x and y; 1.92 GB are still read, since the rows between
+// two bands and the planes between two runs mostly miss L2 (1025 x 513 x 64 complex64:
+// 0.58 -> 0.47 GB for 0.27, 157 -> 125-150 us).
 // NT: y is stored past the caches, which leaves their room to x.
-// 193 x 193 x 97 x 32 complex64: 663 -> 520 us a launch, 3.6 TB/s of x and y.
 // 2-D: one thread per (column position, run of `rows` rows) numbered as above.
 template <typename TI, typename TO, typename TD, int MODE, bool NT>
 __global__ __launch_bounds__(256) void k_march2d(Grid g, const cx<TI>* __restrict__ x,
