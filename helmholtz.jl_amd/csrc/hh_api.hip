@@ -546,19 +546,24 @@ void ensure_work(hh_solver* S, int nrhs) {
   w.nrhs = nrhs;
   w.N = N;
   w.kmax = K;
-  // Node chunks per RHS for the Arnoldi/BiCGSTAB reductions: about 16K blocks
-  // in all (64 per CU, so the last wave of blocks is a small tail), chunks of at
-  // least `least` nodes.  That is 1/1024 of the grid between 256 nodes (one per
-  // thread) and 4096, so one RHS alone still spreads over the chip: with chunks
-  // of 4096 nodes the passes of a 129 x 129 grid ran on 5 blocks (pass 1 at 10
-  // vectors 35 us, pass 2 29 us, against 5.7 and 6.1) and those of 1025 x 513 on
-  // 129 (55 and 58 us against 17 and 20).  It depends on the grid only, not
-  // on the number of RHS, so a small block gives the bits of single solves.  Where
-  // the passes carry a window of 2 n1 extra values of z (complex64 cycle) a chunk
-  // is at least twice that.
+  // Node chunks per RHS for the Arnoldi/BiCGSTAB reductions, by the grid and the
+  // precision alone: the chunks fix the order of every sum, so a column of a block has
+  // the bits of its single solve whatever the block's width or the width these buffers
+  // grew to.  A chunk has 1/1024 of the grid between 256 nodes (one per thread) and
+  // 4096, so one RHS alone still spreads over the chip: with chunks of 4096 nodes the
+  // passes of a 129 x 129 grid ran on 5 blocks (pass 1 at 10 vectors 35 us, pass 2
+  // 29 us, against 5.7 and 6.1) and those of 1025 x 513 on 129 (55 and 58 us against 17
+  // and 20).  Where the passes carry a window of 2 n1 extra values of z (complex64
+  // cycle) a chunk is at least twice that.  Fewer chunks for wide blocks (16384 over all
+  // columns) gain nothing past the run to run spread: whole solves with / without that
+  // limit, 1025 x 513 complex64 x 256 RHS 2404-2436 / 2446 ms, x 48 1206-1207 /
+  // 1205-1208, complex128 x 128 891-893 / 883-884, 193 x 193 x 97 x 32 complex64 1306 /
+  // 1310; and it made one RHS slow after a wide block on the same solver (us an
+  // iteration, with / without: 1025 x 513 after 256 RHS 437-443 / 385-391, 129 x 129
+  // after 1000 RHS 70 / 62.5).
   int64_t least = std::min<int64_t>(4096, std::max<int64_t>(256, ((N + 1023) / 1024 + 255) / 256 * 256));
   if (pr == HH_C64) least = std::min<int64_t>(4096, std::max<int64_t>(least, 4 * (int64_t)S->lv[0].g.n1));
-  int nchunk = (int)std::max<int64_t>(1, std::min<int64_t>((16384 + nrhs - 1) / nrhs, (N + least - 1) / least));
+  int nchunk = (int)std::min<int64_t>(16384, (N + least - 1) / least);
   // 3-D: chunk c is in-plane segment c mod nseg3 over run c / nseg3 of the
   // planes (runs of at least 8 planes) for the H z passes' z march
   w.nseg3 = 0;
