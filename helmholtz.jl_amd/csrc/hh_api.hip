@@ -24,6 +24,7 @@
 
 #include "../../include/helmholtz_amd.h"
 #include "hh_abl.h"
+#include "hh_ahead.h"
 #include "hh_kernels.h"
 #include "hh_unet.h"
 
@@ -264,10 +265,14 @@ struct hh_solver {
   int* conv_d = nullptr;
   double* n2tmp = nullptr;
   double* res_d = nullptr;
-  int* h_done = nullptr;   // pinned host mirrors (h_done: two, taken in turn by the Arnoldi steps)
+  // pinned host mirrors; h_done: done and, est_off(cap) bytes further, est (contiguous on
+  // the device too), two of them, taken in turn by the Arnoldi steps
+  char* h_done = nullptr;
   hipEvent_t ev_done[2] = {nullptr, nullptr};  // h_done's copies have arrived
   int* h_kact = nullptr;
   double* h_res = nullptr;
+  static size_t est_off(int width) { return sizeof(double) * (((size_t)width + 1) / 2); }
+  static size_t done_slot(int width) { return est_off(width) + sizeof(double) * width; }
   double setup_time = 0, solve_time = 0;
   int64_t n_prec = 0;
   // learned coarse-grid correction
@@ -334,7 +339,7 @@ struct hh_solver {
     dfree(V); dfree(Z); dfree(xk); dfree(bk); dfree(wk); dfree(b0);
     V = nullptr; Z = nullptr; xk = bk = wk = nullptr; b0 = nullptr;
     dfree(kw.part); dfree(kw.partn); dfree(kw.h1); dfree(kw.h2); dfree(kw.nrm); dfree(kw.H); dfree(kw.cs);
-    dfree(kw.sn); dfree(kw.gv); dfree(kw.y); dfree(kw.bnorm); dfree(kw.est); dfree(kw.done); dfree(kw.kact);
+    dfree(kw.sn); dfree(kw.gv); dfree(kw.y); dfree(kw.bnorm); dfree(kw.done); dfree(kw.kact);
     dfree(kw.vscale); dfree(kw.fix); dfree(kw.wn2); dfree(kw.h1s); dfree(bsc);
     bsc = nullptr;
     kw = KrylovWork{};
@@ -586,8 +591,8 @@ void ensure_work(hh_solver* S, int nrhs) {
   w.gv = dalloc<cx<double>>((size_t)nrhs * (K + 1));
   w.y = dalloc<cx<double>>((size_t)nrhs * K);
   w.bnorm = dalloc<double>(nrhs);
-  w.est = dalloc<double>(nrhs);
-  w.done = dalloc<int>(nrhs);
+  w.done = (int*)dalloc<char>(hh_solver::done_slot(nrhs));
+  w.est = (double*)((char*)w.done + hh_solver::est_off(nrhs));
   w.kact = dalloc<int>(nrhs);
   w.lazy = pr == HH_C64;
   w.zunscaled = 0;
@@ -601,7 +606,7 @@ void ensure_work(hh_solver* S, int nrhs) {
   S->conv_d = dalloc<int>(nrhs);
   S->n2tmp = dalloc<double>(nrhs);
   S->res_d = dalloc<double>(nrhs);
-  HIPCK(hipHostMalloc((void**)&S->h_done, 2 * sizeof(int) * nrhs, hipHostMallocDefault));
+  HIPCK(hipHostMalloc((void**)&S->h_done, 2 * hh_solver::done_slot(nrhs), hipHostMallocDefault));
   for (hipEvent_t& e : S->ev_done)
     if (!e) HIPCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   HIPCK(hipHostMalloc((void**)&S->h_kact, sizeof(int) * nrhs, hipHostMallocDefault));
@@ -1049,6 +1054,22 @@ void run_fgmres(hh_solver* S, int nrhs, hh_solve_stats* stats) {
   int trial = S->use_learned && !always && S->learn_verdict < 0 ? 0 : -1;
   double rho_learned = 1.0;
   if (S->use_learned) setup_learned(S);
+  // RHS still iterating in h_done's slot i & 1, and the largest estimate among them
+  const size_t flag_bytes = hh_solver::est_off(S->cap) + sizeof(double) * nrhs;
+  auto read_flags = [&](int i, double* worst) {
+    const char* slot = S->h_done + (size_t)(i & 1) * hh_solver::done_slot(S->cap);
+    const int* done = (const int*)slot;
+    const double* est = (const double*)(slot + hh_solver::est_off(S->cap));
+    int active = 0;
+    *worst = 0.0;
+    for (int b = 0; b < nrhs; ++b)
+      if (done[b] == 0) {
+        ++active;
+        *worst = std::max(*worst, est[b]);
+      }
+    return active;
+  };
+  StepAhead rule(tol);
   for (int outer = 0; outer < S->p.max_outer; ++outer) {
     HIPCK(hipMemcpyAsync(S->conv_d, conv.data(), sizeof(int) * nrhs, hipMemcpyHostToDevice, st));
     // plain complex64 cycle: the Arnoldi pass stages the next input and Z
@@ -1061,10 +1082,10 @@ void run_fgmres(hh_solver* S, int nrhs, hh_solve_stats* stats) {
       kr_start_impl<float>(w, S->wk, (cx<float>*)S->V, tol, S->conv_d, S->n2tmp, st);
     else
       kr_start_impl<double>(w, S->wk, S->V, tol, S->conv_d, S->n2tmp, st);
-    HIPCK(hipMemcpyAsync(S->h_done, w.done, sizeof(int) * nrhs, hipMemcpyDeviceToHost, st));
+    HIPCK(hipMemcpyAsync(S->h_done, w.done, flag_bytes, hipMemcpyDeviceToHost, st));
     HIPCK(hipStreamSynchronize(st));
-    int active = 0;
-    for (int b = 0; b < nrhs; ++b) active += S->h_done[b] == 0;
+    double worst = 0.0;
+    int active = read_flags(0, &worst);
     if (active == 0) {
       // every RHS already meets the tolerance at the cycle start
       break;
@@ -1155,26 +1176,25 @@ void run_fgmres(hh_solver* S, int nrhs, hh_solve_stats* stats) {
       }
       HIPCK(hipGraphLaunch(S->gcycle, st));
     } else {
-      // The flags of step j are read while step j + 1 runs, so the queue never drains
-      // between two steps: reading each before the next was launched left the GPU idle
-      // 15-20 us a step (129 x 129, one RHS: 80 us a step).  The step that is launched
-      // past the last needed one finds every flag set and changes nothing.  Steps that
-      // the host itself looks at (captured training pairs, timed launches, the learned
-      // cycle) keep to their order.
+      // A step's flags are read while the next one runs, except where it may be the
+      // last (hh_ahead.h).  A step that is launched past the last one needed finds every
+      // flag set and changes nothing.  Steps that the host itself looks at (captured
+      // training pairs, timed launches, the learned cycle) keep to their order.
       const bool ahead = !S->cap_buf && !S->use_learned && S->kt.kernel == KT_NONE;
-      for (int j = 0; j < K; ++j) {
+      rule.restart(worst);
+      int seen = 0;  // steps whose flags are read
+      for (int j = 0; j < K && active > 0; ++j) {
         S->cap_now = S->cap_buf && nprec_cycle0 + j >= S->cap_lo && nprec_cycle0 + j < S->cap_hi && active == nrhs;
         S->kt_active = active;
         step(j);
-        HIPCK(hipMemcpyAsync(S->h_done + (j & 1) * S->cap, w.done, sizeof(int) * nrhs, hipMemcpyDeviceToHost, st));
+        HIPCK(hipMemcpyAsync(S->h_done + (size_t)(j & 1) * hh_solver::done_slot(S->cap), w.done, flag_bytes,
+                             hipMemcpyDeviceToHost, st));
         HIPCK(hipEventRecord(S->ev_done[j & 1], st));
-        const int seen = ahead ? j - 1 : j;  // the step whose flags are read now
-        if (seen < 0) continue;
-        HIPCK(hipEventSynchronize(S->ev_done[seen & 1]));
-        const int* flags = S->h_done + (seen & 1) * S->cap;
-        active = 0;
-        for (int b = 0; b < nrhs; ++b) active += flags[b] == 0;
-        if (active == 0) break;
+        while (active > 0 && (seen < j || (seen == j && j + 1 < K && (!ahead || rule.may_end())))) {
+          HIPCK(hipEventSynchronize(S->ev_done[seen & 1]));
+          active = read_flags(seen++, &worst);
+          rule.step(worst);
+        }
       }
       finish();
     }
@@ -1370,7 +1390,7 @@ void run_bicgstab(hh_solver* S, int nrhs, hh_solve_stats* stats) {
       HIPCK(hipMemcpyAsync(S->h_done, w.done, sizeof(int) * nrhs, hipMemcpyDeviceToHost, st));
       HIPCK(hipStreamSynchronize(st));
       int left = 0;
-      for (int b = 0; b < nrhs; ++b) left += S->h_done[b] == 0;
+      for (int b = 0; b < nrhs; ++b) left += ((const int*)S->h_done)[b] == 0;
       if (left == 0) break;
     }
     HIPCK(hipMemcpyAsync(S->h_kact, w.kact, sizeof(int) * nrhs, hipMemcpyDeviceToHost, st));
