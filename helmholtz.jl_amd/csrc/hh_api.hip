@@ -1589,12 +1589,10 @@ void op_apply_device(hh_op* op, double shift, const void* xin, void* yout, int64
                                        nullptr, (cx<double>*)yout, op->d64, mm, sfac, nullptr, op->stream);
   } else if (prec == HH_C128)
     launch_stencil<double, double, double, M_APPLY>(op->g, (int)nrhs, (const cx<double>*)xin, nullptr,
-                                                    (cx<double>*)yout, op->d64, mm, sfac, 0.0, nullptr, op->stream, 0,
-                                                    nullptr, true);
+                                                    (cx<double>*)yout, op->d64, mm, sfac, 0.0, nullptr, op->stream);
   else
     launch_stencil<float, float, float, M_APPLY>(op->g, (int)nrhs, (const cx<float>*)xin, nullptr,
-                                                 (cx<float>*)yout, op->d32, mm, sfac, 0.0, nullptr, op->stream, 0, nullptr,
-                                                 true);
+                                                 (cx<float>*)yout, op->d32, mm, sfac, 0.0, nullptr, op->stream);
   HIPCK(hipGetLastError());
 }
 }  // namespace

@@ -16,7 +16,6 @@
 #include "hh_kernels.h"
 
 #include <algorithm>
-#include <type_traits>
 
 namespace hh {
 
@@ -182,16 +181,6 @@ struct XEdge {
   }
 };
 
-template <bool NT, typename T>
-__device__ __forceinline__ void put(cx<T>* q, cx<T> v) {
-  typedef T v2 __attribute__((ext_vector_type(2)));
-  const v2 u = {v.re, v.im};
-  if (NT)
-    __builtin_nontemporal_store(u, (v2*)q);
-  else
-    *(v2*)q = u;
-}
-
 // Larger blocks: the gathering kernels above load five (2-D: three) values of x a node
 // and read a plane's neighbours a step after the plane itself, when part of it has left
 // L1 and L2: 193 x 193 x 97 x 32 complex64 took 55.7 million L2 requests and read 2.03 GB
@@ -201,9 +190,8 @@ __device__ __forceinline__ void put(cx<T>* q, cx<T> v) {
 // requests, 520 us, 3.6 TB/s of x and y; 1.92 GB are still read, since the rows between
 // two bands and the planes between two runs mostly miss L2 (1025 x 513 x 64 complex64:
 // 0.58 -> 0.47 GB for 0.27, 157 -> 125-150 us).
-// NT: y is stored past the caches, which leaves their room to x.
 // 2-D: one thread per (column position, run of `rows` rows) numbered as above.
-template <typename TI, typename TO, typename TD, int MODE, bool NT>
+template <typename TI, typename TO, typename TD, int MODE>
 __global__ __launch_bounds__(256) void k_march2d(Grid g, const cx<TI>* __restrict__ x,
                                                    const cx<TO>* __restrict__ b, cx<TO>* __restrict__ y,
                                                    const cx<TD>* __restrict__ d, const double* __restrict__ m,
@@ -246,7 +234,7 @@ __global__ __launch_bounds__(256) void k_march2d(Grid g, const cx<TI>* __restric
     const cx<TD> Ax = apply5(c, cvt<TI, TD>(xl), cvt<TI, TD>(xrr), cvt<TI, TD>(xm), cvt<TI, TD>(xp), ih1, ih2, dv);
     cx<TD> Dtot = dv;
     if (MODE == M_JACOBI && !fj) Dtot.re += ldx + (TD)(g.ih2 * lap_diag1(j, n2, g.bc));
-    if (own && j0 + s < n2) put<NT>(yo + p, finish<TO, TD, MODE>(c, Ax, bv, Dtot, wj, fj != nullptr, fv));
+    if (own && j0 + s < n2) yo[p] = finish<TO, TD, MODE>(c, Ax, bv, Dtot, wj, fj != nullptr, fv);
     xm = xc;
     xc = xp;
     ec = ep;
@@ -256,7 +244,7 @@ __global__ __launch_bounds__(256) void k_march2d(Grid g, const cx<TI>* __restric
 // 3-D: a thread owns RY nodes of one in-plane column, rows j0 .. j0 + RY - 1, over a
 // run of `rows` planes; the columns of a band of RY rows are numbered consecutively
 // over the bands.
-template <typename TI, typename TO, typename TD, int MODE, int RY, bool NT>
+template <typename TI, typename TO, typename TD, int MODE, int RY>
 __global__ __launch_bounds__(256) void k_march3d(Grid g, const cx<TI>* __restrict__ x,
                                                    const cx<TO>* __restrict__ b, cx<TO>* __restrict__ y,
                                                    const cx<TD>* __restrict__ d, const double* __restrict__ m,
@@ -333,7 +321,7 @@ __global__ __launch_bounds__(256) void k_march3d(Grid g, const cx<TI>* __restric
       if (MODE == M_JACOBI && !fj)
         Dtot.re += (TD)(ldx + (TD)(g.ih2 * lap_diag1(j0 + r, n2, g.bc))) + (TD)(g.ih3 * lap_diag1(k, n3, g.bc));
       if (own && j0 + r < n2)
-        put<NT>(yo + pl + rw[r + 1] + i, finish<TO, TD, MODE>(c, Ax, bv[r], Dtot, wj, fj != nullptr, fv[r]));
+        yo[pl + rw[r + 1] + i] = finish<TO, TD, MODE>(c, Ax, bv[r], Dtot, wj, fj != nullptr, fv[r]);
     }
 #pragma unroll
     for (int r = 0; r < RY; ++r) {
@@ -850,19 +838,23 @@ static inline int pick_rows(int len, int64_t cols) {
 }
 
 // x blocks up to 16 MB lie in the L2s, where re-reading the neighbours is cheaper than
-// the marches' longer start: 129 x 129 x 1 complex128 14.4 / 15.1 us a call (gathered /
-// marched), 61 x 50 x 33 x 8 complex64 18.4 / 19.7, 270 x 42 x 82 complex128 19.6 / 20.1.
-// Beyond: 513 x 257 x 8 complex128 20.7 / 19.7 us, 97 x 97 x 49 x 8 complex64 31.1 / 29.8,
-// 1025 x 513 x 64 complex64 167 / 133, 193 x 193 x 97 x 32 complex64 673 / 528,
-// x 12 complex128 504 / 380.  RY: complex128 2 / 4 rows 37 / 41 us (101 x 83 x 57 x 8),
-// complex64 566 / 528 us (193 x 193 x 97 x 32).  Stores past the caches (stream_out: y is
-// the caller's) help while x fits in about two Infinity Caches: 97 x 97 x 49 x 64
-// complex64 165 -> 115 us, 150 x 171 x 101 x 3 complex128 82 -> 71; with 925 MB of x
-// they cost 528 -> 551.
+// the marches' longer start: us a call on an x of its own each time, gathered / marched,
+// 129 x 129 x 1 complex128 19.3 / 20.6, 61 x 50 x 33 x 8 complex64 23.4 / 26.3, 1025 x 513
+// x 2 complex128 (16 MB) 26.5 / 27.5.  From there on the marches gain: 97 x 97 x 49 x 3
+// complex128 (21 MB) 31.6 / 30.8, x 8 complex64 (28 MB) 42.8 / 41.7, 150 x 171 x 101 x 3
+// complex128 105 / 88, 1025 x 513 x 64 complex64 171 / 149, 193 x 193 x 97 x 12 complex128
+// 510 / 387, x 32 complex64 680 / 535.  RY: complex128 2 / 4 rows 37 / 41 us (101 x 83 x
+// 57 x 8), complex64 566 / 528 us (193 x 193 x 97 x 32).
+// y goes through the caches.  Stored past them the call is faster only on 96-256 MB of x
+// that the last call left in the Infinity Cache (97 x 97 x 49 x 55 complex64 152 -> 117
+// us; an x of its own each time 153 / 154), and the kernel that reads y next pays for it
+// (call and a product of y, through / past: 513 x 257 x 64 complex64 85 / 103 us, x 32
+// complex128 82 / 91, 97 x 97 x 49 x 142 complex64 699 / 743; call and a scaling of y, an x
+// of its own each time: from 0.5% faster to 7% slower past them, 2% slower in the mean).
 template <typename TI, typename TO, typename TD, int MODE>
 void launch_stencil(const Grid& g, int nrhs, const cx<TI>* x, const cx<TO>* b, cx<TO>* y, const cx<TD>* d,
                     const double* m, cx<double> sfac, double wj, const int* skip, hipStream_t s, int rows_override,
-                    const cx<TD>* fj, bool stream_out) {
+                    const cx<TD>* fj) {
   const bool d3 = g.dim == 3;
   const int len = d3 ? g.n3 : g.n2;
   const int64_t xbytes = (int64_t)sizeof(cx<TI>) * g.N * nrhs;
@@ -888,52 +880,46 @@ void launch_stencil(const Grid& g, int nrhs, const cx<TI>* x, const cx<TO>* b, c
   const int runs = (len + rows - 1) / rows;
   const int64_t items = (int64_t)g.n1 * (d3 ? bands : runs);
   const TileMap tm = make_tile_map((int)((items + 255) / 256), d3 ? runs : 1, nrhs);
-  auto go = [&](auto nt) {
-    constexpr bool NT = decltype(nt)::value;
-    if (d3)
-      hipLaunchKernelGGL((k_march3d<TI, TO, TD, MODE, RY, NT>), dim3(tm.T), dim3(256), 0, s, g, x, b, y, d, m, sfac,
-                         (TD)wj, rows, tm, skip, fj);
-    else
-      hipLaunchKernelGGL((k_march2d<TI, TO, TD, MODE, NT>), dim3(tm.T), dim3(256), 0, s, g, x, b, y, d, m, sfac,
-                         (TD)wj, rows, tm, skip, fj);
-  };
-  if constexpr (MODE == M_APPLY)
-    if (stream_out && xbytes <= (512 << 20)) return go(std::true_type{});
-  go(std::false_type{});
+  if (d3)
+    hipLaunchKernelGGL((k_march3d<TI, TO, TD, MODE, RY>), dim3(tm.T), dim3(256), 0, s, g, x, b, y, d, m, sfac, (TD)wj,
+                       rows, tm, skip, fj);
+  else
+    hipLaunchKernelGGL((k_march2d<TI, TO, TD, MODE>), dim3(tm.T), dim3(256), 0, s, g, x, b, y, d, m, sfac, (TD)wj,
+                       rows, tm, skip, fj);
 }
 
 template void launch_stencil<double, double, double, M_APPLY>(const Grid&, int, const cx<double>*,
                                                                const cx<double>*, cx<double>*,
                                                                const cx<double>*, const double*, cx<double>,
                                                                double, const int*, hipStream_t, int,
-                                                              const cx<double>*, bool);
+                                                              const cx<double>*);
 template void launch_stencil<double, double, double, M_RESID>(const Grid&, int, const cx<double>*,
                                                                const cx<double>*, cx<double>*,
                                                                const cx<double>*, const double*, cx<double>,
                                                                double, const int*, hipStream_t, int,
-                                                              const cx<double>*, bool);
+                                                              const cx<double>*);
 template void launch_stencil<double, double, double, M_JACOBI>(const Grid&, int, const cx<double>*,
                                                                 const cx<double>*, cx<double>*,
                                                                 const cx<double>*, const double*, cx<double>,
                                                                 double, const int*, hipStream_t, int,
-                                                              const cx<double>*, bool);
+                                                              const cx<double>*);
 template void launch_stencil<float, float, float, M_APPLY>(const Grid&, int, const cx<float>*, const cx<float>*,
                                                             cx<float>*, const cx<float>*, const double*,
                                                             cx<double>, double, const int*, hipStream_t, int,
-                                                              const cx<float>*, bool);
+                                                              const cx<float>*);
 template void launch_stencil<float, float, float, M_RESID>(const Grid&, int, const cx<float>*, const cx<float>*,
                                                             cx<float>*, const cx<float>*, const double*,
                                                             cx<double>, double, const int*, hipStream_t, int,
-                                                              const cx<float>*, bool);
+                                                              const cx<float>*);
 template void launch_stencil<float, float, float, M_JACOBI>(const Grid&, int, const cx<float>*, const cx<float>*,
                                                              cx<float>*, const cx<float>*, const double*,
                                                              cx<double>, double, const int*, hipStream_t, int,
-                                                              const cx<float>*, bool);
+                                                              const cx<float>*);
 template void launch_stencil<float, double, double, M_APPLY>(const Grid&, int, const cx<float>*,
                                                               const cx<double>*, cx<double>*,
                                                               const cx<double>*, const double*, cx<double>,
                                                               double, const int*, hipStream_t, int,
-                                                              const cx<double>*, bool);
+                                                              const cx<double>*);
 
 template <typename T>
 void launch_jacobi0(const Grid& g, int nrhs, const cx<T>* b, cx<T>* x, const cx<T>* f, const int* skip,
