@@ -494,13 +494,14 @@ void setup_learned(hh_solver* S) {
 // row-major A^-1 of the coarsest level (left half of the Gauss-Jordan workspace)
 const cx<double>* coarse_inv(hh_solver* S) { return S->coarse_aug; }
 
-// coarsest-level solve x = A^-1 r (MFMA in the complex64 mode)
+// coarsest-level solve x = A^-1 r (complex64: on MFMA, from the packed inverse that every
+// complex64 hierarchy holds)
 template <typename T>
 void coarse_apply(hh_solver* S, int64_t n, int nrhs, const cx<T>* r, cx<T>* x, const int* skip, hipStream_t st) {
-  if (std::is_same<T, float>::value && S->coarse_pack)
-    launch_dense_apply_mfma(S->coarse_pack, n, nrhs, (const cx<float>*)r, (cx<float>*)x, skip, st);
+  if constexpr (std::is_same<T, float>::value)
+    launch_dense_apply_mfma(S->coarse_pack, n, nrhs, r, x, skip, st);
   else
-    launch_dense_apply<T>(coarse_inv(S), n, nrhs, r, x, skip, st);
+    launch_dense_apply(coarse_inv(S), n, nrhs, r, x, skip, st);
 }
 
 void ensure_work(hh_solver* S, int nrhs) {

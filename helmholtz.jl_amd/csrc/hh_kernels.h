@@ -39,9 +39,8 @@ void launch_add_const(double* a, double c, int64_t n, hipStream_t s);
 // leaves A^-1 row-major in M[0, n*n); M[n*n, 2*n*n) and work (dense_inverse_work_bytes(n) bytes) are its workspace
 size_t dense_inverse_work_bytes(int64_t n);
 void launch_dense_inverse(const Grid& g, const cx<double>* d, cx<double>* M, void* work, hipStream_t s);
-template <typename T>
-void launch_dense_apply(const cx<double>* Ainv, int64_t n, int nrhs, const cx<T>* r, cx<T>* x, const int* skip,
-                        hipStream_t s);
+void launch_dense_apply(const cx<double>* Ainv, int64_t n, int nrhs, const cx<double>* r, cx<double>* x,
+                        const int* skip, hipStream_t s);
 // complex64 coarsest apply on MFMA: P = the inverse packed by pack_inv_mfma (fp32, pack_inv_mfma_size(n) floats)
 void pack_inv_mfma(const cx<double>* Ainv, int64_t n, float* P, hipStream_t s);
 int64_t pack_inv_mfma_size(int64_t n);

@@ -632,9 +632,9 @@ __device__ __forceinline__ cx<double> cmac(cx<double> acc, cx<double> a, cx<doub
   return mk<double>(fma(-a.im, r.im, fma(a.re, r.re, acc.re)), fma(a.im, r.re, fma(a.re, r.im, acc.im)));
 }
 
-template <typename T, int RT, int DR, int UN>
+template <int RT, int DR, int UN>
 __global__ __launch_bounds__(256) void k_dense_apply(const cx<double>* __restrict__ Arow, int n, int nrhs,
-                                                     const cx<T>* __restrict__ r, cx<T>* __restrict__ x,
+                                                     const cx<double>* __restrict__ r, cx<double>* __restrict__ x,
                                                      const int* __restrict__ skip) {
   constexpr int M = 2 * RT * DR;
   __shared__ double sums[4][M];
@@ -651,7 +651,7 @@ __global__ __launch_bounds__(256) void k_dense_apply(const cx<double>* __restric
   const cx<double>* row[RT];
 #pragma unroll
   for (int a = 0; a < RT; ++a) row[a] = Arow + (int64_t)min(i0 + a, n - 1) * n;
-  const cx<T>* rc[DR];
+  const cx<double>* rc[DR];
 #pragma unroll
   for (int k = 0; k < DR; ++k) rc[k] = r + (int64_t)(rhs0 + min(k, nr - 1)) * n;
   cx<double> acc[RT][DR];
@@ -661,7 +661,7 @@ __global__ __launch_bounds__(256) void k_dense_apply(const cx<double>* __restric
     for (int k = 0; k < DR; ++k) acc[a][k] = mk<double>(0.0, 0.0);
   for (int j = threadIdx.x; j < n; j += 256 * UN) {
     cx<double> av[UN][RT];
-    cx<T> rv[UN][DR];
+    cx<double> rv[UN][DR];
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
       const int ju = min(j + 256 * u, n - 1);  // a column past the last one: its values times 0
@@ -674,7 +674,7 @@ __global__ __launch_bounds__(256) void k_dense_apply(const cx<double>* __restric
     for (int u = 0; u < UN; ++u)
 #pragma unroll
       for (int k = 0; k < DR; ++k) {
-        const cx<double> rk = j + 256 * u < n ? cvt<T, double>(rv[u][k]) : mk<double>(0.0, 0.0);
+        const cx<double> rk = j + 256 * u < n ? rv[u][k] : mk<double>(0.0, 0.0);
 #pragma unroll
         for (int a = 0; a < RT; ++a) acc[a][k] = cmac(acc[a][k], av[u][a], rk);
       }
@@ -693,8 +693,8 @@ __global__ __launch_bounds__(256) void k_dense_apply(const cx<double>* __restric
   if (q >= M) return;
   const int a = (q >> 1) / DR, k = (q >> 1) % DR;
   if (i0 + a >= n || k >= nr || (skip && skip[rhs0 + k])) return;
-  ((T*)x)[2 * ((int64_t)(rhs0 + k) * n + i0 + a) + (q & 1)] =
-      (T)(((sums[0][q] + sums[1][q]) + sums[2][q]) + sums[3][q]);
+  ((double*)x)[2 * ((int64_t)(rhs0 + k) * n + i0 + a) + (q & 1)] =
+      ((sums[0][q] + sums[1][q]) + sums[2][q]) + sums[3][q];
 }
 
 // ---- coarsest apply on MFMA (complex64 preconditioner) ----
@@ -1014,11 +1014,11 @@ void launch_add_const(double* a, double c, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_add_const, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, c, n);
 }
 
-template <typename T, int RT, int DR, int UN>
-static void dense_apply_go(const cx<double>* Ainv, int n, int nrhs, const cx<T>* r, cx<T>* x, const int* skip,
-                           hipStream_t s) {
+template <int RT, int DR, int UN>
+static void dense_apply_go(const cx<double>* Ainv, int n, int nrhs, const cx<double>* r, cx<double>* x,
+                           const int* skip, hipStream_t s) {
   dim3 grid((unsigned)((n + RT - 1) / RT), (unsigned)((nrhs + DR - 1) / DR));
-  hipLaunchKernelGGL((k_dense_apply<T, RT, DR, UN>), grid, dim3(256), 0, s, Ainv, n, nrhs, r, x, skip);
+  hipLaunchKernelGGL((k_dense_apply<RT, DR, UN>), grid, dim3(256), 0, s, Ainv, n, nrhs, r, x, skip);
 }
 
 // Rows x right-hand sides per block.  Kernel times on MI355X in us, one-row (4 x 4)
@@ -1031,29 +1031,24 @@ static void dense_apply_go(const cx<double>* Ainv, int n, int nrhs, const cx<T>*
 // 22.7).  Past the Infinity Cache (n > 4096) the inverse comes from HBM, and four rows with
 // more columns in flight keep it busiest: 6305 nodes with the call 1 RHS 131 / 120 us,
 // 2 RHS 132 / 125, 4 RHS 147 / 140, 8 RHS 269 / 254.
-template <typename T>
-void launch_dense_apply(const cx<double>* Ainv, int64_t n, int nrhs, const cx<T>* r, cx<T>* x, const int* skip,
-                        hipStream_t s) {
+void launch_dense_apply(const cx<double>* Ainv, int64_t n, int nrhs, const cx<double>* r, cx<double>* x,
+                        const int* skip, hipStream_t s) {
   if (n > 4096) {
     if (nrhs == 1)
-      dense_apply_go<T, 2, 1, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
+      dense_apply_go<2, 1, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
     else if (nrhs == 2)
-      dense_apply_go<T, 4, 2, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
+      dense_apply_go<4, 2, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
     else
-      dense_apply_go<T, 4, 4, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
+      dense_apply_go<4, 4, 4>(Ainv, (int)n, nrhs, r, x, skip, s);
   } else if (nrhs == 1) {
-    dense_apply_go<T, 2, 1, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
+    dense_apply_go<2, 1, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
   } else if (nrhs == 2) {
-    dense_apply_go<T, 2, 2, 2>(Ainv, (int)n, nrhs, r, x, skip, s);
+    dense_apply_go<2, 2, 2>(Ainv, (int)n, nrhs, r, x, skip, s);
   } else if (nrhs <= 4 || n <= 1600) {
-    dense_apply_go<T, 2, 4, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
+    dense_apply_go<2, 4, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
   } else {
-    dense_apply_go<T, 2, 8, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
+    dense_apply_go<2, 8, 1>(Ainv, (int)n, nrhs, r, x, skip, s);
   }
 }
-template void launch_dense_apply<double>(const cx<double>*, int64_t, int, const cx<double>*, cx<double>*,
-                                         const int*, hipStream_t);
-template void launch_dense_apply<float>(const cx<double>*, int64_t, int, const cx<float>*, cx<float>*,
-                                        const int*, hipStream_t);
 
 }  // namespace hh
