@@ -174,9 +174,10 @@ __device__ __forceinline__ void tile_of(const TileMap& m, int& xt, int& yt, int&
 
 // Sums of M values over a wavefront, the values shared out among the lanes as
 // the reduction narrows: at each step a lane keeps one half of its values and
-// hands the other half to its partner, so M = 21 takes 23 exchanges where M
+// hands the other half to its partner, so M = 21 takes 24 exchanges where M
 // separate reductions take 126 (the same tree of additions, the same bits).
-// On return v[0 .. K) holds the sums of values base .. base + valid - 1.
+// put(i, sum) receives the sum of value i, once, in the lane that ends with it; v
+// holds the values base .. base + valid - 1 (at the call 0 and M).
 template <int M, int O>
 struct WaveSums {
   static constexpr int Hf = (M + 1) / 2;

@@ -30,7 +30,8 @@
 // reads, 1.4-1.8 us a column), the rows used before take one small product (k_gj_rows),
 // and the rank-32 update stops at column ke + 2 bw.  Panel form / this one: 1183 nodes
 // (13 x 13 x 7) 6.7 / 4.5 ms, 2145 nodes 16.8 / 8.1 ms, 3201 nodes 32 / 15 ms, 8385
-// nodes 371 / 116 ms; 561 nodes 1.9 / 1.8 ms.
+// nodes 371 / 116 ms; 561 nodes 1.9 / 1.8 ms.  The node order is the grid's own, so a 2-D
+// grid of n1 > 224 takes the panels although its other axis may be short.
 #include <algorithm>
 
 #include "hh_kernels.h"
@@ -122,7 +123,7 @@ __device__ __forceinline__ unsigned long long wave_max(unsigned long long v) {
 // column kb + s of the block the panel belongs to; pin: the panel's exchange,
 // pout (with the block's last panel, else null): the whole block's exchange.
 // A pivot is found as the maximum of one 64-bit key per row, |a|^2 with its 14
-// lowest bits (6e-13 of it, n < 2^14) replaced by the reversed row number: one
+// lowest bits (up to 3.6e-12 of it, n < 2^14) replaced by the reversed row number: one
 // DPP reduction and one LDS atomic per wavefront (a 4-column panel of 2145 rows:
 // 20 us with value and row reduced by shuffles, 15 us so).
 template <int W, int R>

@@ -471,9 +471,13 @@ struct Runs3 {
   int ytiles, zrun;
   TileMap m;
 };
-// A complex128 block takes a CU for itself (LDS, 88-94 VGPRs), so more than 256 blocks
-// only recompute more planes: 97 x 97 x 49 x 8, one W cycle 497 us with at least
-// 256 blocks, 534 with 512, 560 with 1024 (145 x 113 x 65 x 3: 722 / 704 / 688).
+// A complex128 block takes a CU for itself (LDS, 88-94 VGPRs): more than 256 blocks
+// recompute more planes and gain only where 256 blocks and a few leave a long tail.
+// Neither is the better one everywhere.  One W cycle in us with at least 256 / 512 / 1024
+// blocks: 97 x 97 x 49 x 8 507 / 543 / 571, x 32 1369 / 1408 / 1408, 145 x 145 x 81 x 1 735 /
+// 790 / 789; 145 x 113 x 65 x 3 733 / 715 / 700, 145 x 145 x 81 x 4 1400 / 1344 / 1282, 113 x
+// 65 x 57 x 6 608 / 595 / 597; the same within 1% on 97 x 97 x 49 x 1, 81 x 65 x 41 x 4,
+// 129 x 65 x 33 x 5, 49 x 49 x 25 x 8 and 33 x 33 x 25 x 8.
 Runs3 runs3(const Grid& g, int nrhs, int H, bool c128) {
   const int target = c128 ? 256 : 1024;
   Runs3 r;

@@ -21,8 +21,8 @@
 // sum).  The levels this runs on are small, so a smoothing costs its launches:
 // one kernel per operation (F v, A u, dots, reduction, update, scaling) took 27 for
 // two steps, with the dots on one block per 4096 nodes (8.9 us each); now eight.
-// K-cycle solve of 257 x 129 x 4 RHS in complex128 (94 iterations of 3 levels) on
-// MI355X: 83 ms with the separate kernels, 41 ms.
+// K-cycle solve of 257 x 129 x 4 RHS in complex128 (3 levels; 89 to 95 iterations by
+// the medium) on MI355X: 83 ms with the separate kernels, 41 ms.
 #include "hh_kernels.h"
 
 #include <algorithm>

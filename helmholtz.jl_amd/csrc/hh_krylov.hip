@@ -23,7 +23,7 @@
 // complex64 w' is then the preconditioner's next input as it is.
 // Partial sums are per (chunk, RHS) and reduced in a fixed order, so results
 // are bit-reproducible run to run.  The small Hessenberg/Givens work runs on
-// the device (one wavefront per RHS) so a whole iteration needs no host sync.
+// the device (one block per RHS) so a whole iteration needs no host sync.
 #include "hh_kernels.h"
 
 namespace hh {

@@ -734,8 +734,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // its four wavefronts take every fourth K-group and their partial tiles are
 // summed through LDS in a fixed order (deterministic).  Bound by the address unit: a B
 // operand is 16 columns apart for 16 lanes, so it is one 16-byte load of four k and not
-// two of 8 (561 nodes x 256 RHS 34.8 -> 17.0 us, 1183 x 32 28.4 -> 20.4, 2145 x 256
-// 391 -> 195, 97 TFLOP/s; gfx950 takes 16-byte loads at 8-byte alignment).
+// two of 8 (561 nodes x 256 RHS 34.8 -> 17.0 us, 2145 x 256 391 -> 195, 97 TFLOP/s, 1183 x
+// 32 28.4 -> 20.4 and with two K-groups in flight 13.1; gfx950 takes 16-byte loads at
+// 8-byte alignment).
 template <int UN>
 __global__ __launch_bounds__(256) void k_dense_apply_mfma(const float4* __restrict__ P, int n2, int ng, int nrhs,
                                                           const float* __restrict__ r, float* __restrict__ x,
