@@ -561,12 +561,11 @@ void ensure_work(hh_solver* S, int nrhs) {
   // 29 us, against 5.7 and 6.1) and those of 1025 x 513 on 129 (55 and 58 us against 17
   // and 20).  Where the passes carry a window of 2 n1 extra values of z (complex64
   // cycle) a chunk is at least twice that.  Fewer chunks for wide blocks (16384 over all
-  // columns) gain nothing past the run to run spread: whole solves with / without that
-  // limit, 1025 x 513 complex64 x 256 RHS 2404-2436 / 2446 ms, x 48 1206-1207 /
-  // 1205-1208, complex128 x 128 891-893 / 883-884, 193 x 193 x 97 x 32 complex64 1306 /
-  // 1310; and it made one RHS slow after a wide block on the same solver (us an
-  // iteration, with / without: 1025 x 513 after 256 RHS 437-443 / 385-391, 129 x 129
-  // after 1000 RHS 70 / 62.5).
+  // columns) gain little: whole solves with / without that limit, 1025 x 513 complex64 x
+  // 256 RHS 8.96 / 9.02 ms/RHS, x 48 1206-1207 / 1205-1208 ms, complex128 x 128 891-893 /
+  // 883-884, 193 x 193 x 97 x 32 complex64 1306 / 1310; and it made one RHS slow after a
+  // wide block on the same solver (us an iteration, with / without: 1025 x 513 after 256
+  // RHS 437-443 / 385-391, 129 x 129 after 1000 RHS 70 / 62.5).
   int64_t least = std::min<int64_t>(4096, std::max<int64_t>(256, ((N + 1023) / 1024 + 255) / 256 * 256));
   if (pr == HH_C64) least = std::min<int64_t>(4096, std::max<int64_t>(least, 4 * (int64_t)S->lv[0].g.n1));
   int nchunk = (int)std::min<int64_t>(16384, (N + least - 1) / least);
